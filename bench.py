@@ -37,7 +37,8 @@ HBM_PEAK_GBS = 8000.0
 # source files that define the headline kNN kernel; the committed counter
 # summary records their hash, and its traffic figure is used only while
 # the hash still matches
-KNN_KERNEL_SOURCES = ("cudakdtree_amd/csrc/query_impl.h", "cudakdtree_amd/csrc/query_inst.hip",
+KNN_KERNEL_SOURCES = ("cudakdtree_amd/csrc/query_impl.h", "cudakdtree_amd/csrc/query_box.h",
+                      "cudakdtree_amd/csrc/query_inst.hip",
                       "cudakdtree_amd/csrc/cukd_common.h", "include/cukd/traverse.h",
                       "include/cukd/knn.h", "include/cukd/fcp.h", "cudakdtree_amd/build.py")
 

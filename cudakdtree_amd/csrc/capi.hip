@@ -281,7 +281,8 @@ struct TuneKey {
   }
 };
 struct TuneVal {
-  int block, sort, lanes;
+  int block, sort;
+  bool box;
 };
 std::mutex g_tune_mu;
 std::map<TuneKey, TuneVal> g_tune;
@@ -307,14 +308,8 @@ static int run_queries(QueryArgs a, int D, int traversal, int flags, const MemRe
                        void *order_ws, size_t order_ws_bytes, bool repeatable,
                        hipStream_t stream, const char *what)
 {
-  TuneVal cfg{128, (flags & CUKD_QUERY_SORT) ? 1 : 0, (flags & CUKD_QUERY_ONE_PER_LANE) ? 1 : 2};
-  // two queries per lane: stack-based, registers-only lists, round-robin
-  // dims, node offsets within 32 bits
-  const bool two_ok = traversal == CUKD_STACK_BASED && a.t.dim_offset < 0 &&
-                      (a.fq.seg_off ? a.tree_bytes : (uint64_t)a.t.n * (uint64_t)a.t.stride) <=
-                          0xffffffffull &&
-                      (a.list_kind < 0 || (a.list_kind == CUKD_LIST_FIXED &&
-                                           (a.k == 1 || a.k == 4 || a.k == 8 || a.k == 16)));
+  TuneVal cfg{0, (flags & CUKD_QUERY_SORT) ? 1 : 0, !(flags & CUKD_QUERY_ONE_PER_LANE)};
+  const bool two_ok = box_ok(a);
   bool tune = false;
   TuneKey key;
   memset(&key, 0, sizeof(key));
@@ -349,12 +344,12 @@ static int run_queries(QueryArgs a, int D, int traversal, int flags, const MemRe
     float best = 3.4e38f;
     TuneVal bestv = cfg;
     const int blocks[3] = {64, 128, 256};
-    for (int lanes = 1; lanes <= (two_ok ? 2 : 1) && e == hipSuccess; lanes++)
+    for (int box = 0; box <= (two_ok ? 1 : 0) && e == hipSuccess; box++)
     for (int sort = 0; sort < 2 && e == hipSuccess; sort++)
       for (int bi = 0; bi < 3 && e == hipSuccess; bi++) {
         QueryArgs v = a;
         v.block = blocks[bi];
-        v.lanes = lanes;
+        v.box = box != 0;
         v.stats = nullptr;  // statistics count the final launch only
         for (int rep = 0; rep < 3 && e == hipSuccess; rep++) {
           if (rep == 1) e = hipEventRecord(e0, stream);
@@ -367,7 +362,7 @@ static int run_queries(QueryArgs a, int D, int traversal, int flags, const MemRe
         if (e == hipSuccess) e = hipEventElapsedTime(&ms, e0, e1);
         if (e == hipSuccess && ms < best) {
           best = ms;
-          bestv = TuneVal{blocks[bi], sort, lanes};
+          bestv = TuneVal{blocks[bi], sort, box != 0};
         }
       }
     if (e0) (void)hipEventDestroy(e0);
@@ -380,7 +375,7 @@ static int run_queries(QueryArgs a, int D, int traversal, int flags, const MemRe
   }
   if (e == hipSuccess) {
     a.block = cfg.block;
-    a.lanes = two_ok ? cfg.lanes : 1;
+    a.box = cfg.box;
     a.presorted = (flags & CUKD_QUERY_PRESORTED) != 0;
     a.order = cfg.sort ? make_query_order(otmp, a.queries, a.nq, D, stream) : nullptr;
     e = launch_query(D, traversal, a, stream);

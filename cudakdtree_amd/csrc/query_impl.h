@@ -1,10 +1,10 @@
 // query_impl.h -- batched FCP / kNN kernels over a left-balanced k-d tree.
 //
-// One query per lane.  The traversals and result types are the public
-// device-inline ones of include/cukd/ (traverse.h, fcp.h, knn.h), run
-// through an accessor over the run-time element layout, so the batched
-// path and user kernels share one implementation; ids and dist2 bits
-// equal the CPU oracle's, ties included.
+// One query per lane.  k_query runs the public device-inline traversals of
+// include/cukd/ (traverse.h, fcp.h, knn.h) through an accessor over the
+// run-time element layout; k_query_box (query_box.h), the default over trees
+// with round-robin split dims, gives the same results with fewer visits.
+// ids and dist2 bits equal the CPU oracle's, ties included.
 #pragma once
 #pragma clang fp contract(off)
 
@@ -354,324 +354,11 @@ __global__ __launch_bounds__(256) void k_query(TreeView t, const float *queries,
   if (stats) atomicAdd(stats, (unsigned long long)visits);
 }
 
-// ---------------------------------------------------------------------------
-// batch kernel: two stack-based queries per lane
-// ---------------------------------------------------------------------------
-// The stack-based traversal is a chain of dependent node loads, and a
-// wave holds at most one load per lane in flight.  Here each lane steps
-// two queries together: every iteration issues the node loads of both
-// before using either, so twice as many loads are in flight per wave slot
-// for little more than one query's registers.  Each query's steps are
-// those of traverse_stack_based (include/cukd/traverse.h), one node load
-// per step:
-//   descend  visit node curr, mark its far child pending if the plane is
-//            within the cull distance, go to the close child; past the
-//            last node, pop
-//   pop      re-read the parent of the deepest pending far child and enter
-//            that child if its plane is within the cull distance, else pop
-//            the next one
-// so every query visits the same nodes in the same order with the same
-// candidate updates, and its result is bit-identical to one query per lane.
-//
-// The step is written for few vector instructions, since a wave executes
-// every path some lane takes: node byte offsets are 32-bit (trees under
-// 4 GiB) and follow the descent by doubling, the level is counted rather
-// than recomputed, and descend and pop share the plane test.
-enum { SB_DESCEND = 0, SB_POP = 1, SB_DONE = 2 };
+}  // namespace cukd_amd
 
-// round-robin split dim of level l (0 <= l < 32)
-template <int D>
-__device__ inline int rr_dim(int l)
-{
-  if ((D & (D - 1)) == 0) return l & (D - 1);
-  if (D == 3) return l - (int)__umul24((unsigned)__umul24((unsigned)l, 11u) >> 5, 3u);  // l / 3 for l < 32
-  return l % D;
-}
+#include "query_box.h"
 
-struct SbSlot {
-  int mode;
-  int curr;          // descend: node to visit; pop: end of the path (>= n)
-  int lvl;           // level of curr
-  int pd;            // pop: depth of the far child being tested
-  unsigned off;      // byte offset of the node loaded next (curr, or the far child's parent)
-  unsigned pending;  // bit d: the far child at depth d of the path is still to be visited
-  float cull;
-};
-
-template <int D, class R>
-__device__ inline void sb_step(R &res, const float (&q)[D], const float (&p)[D], int n,
-                               unsigned stride, SbSlot &s, unsigned &visits)
-{
-  if (s.mode == SB_DONE) return;
-  const bool desc = s.mode == SB_DESCEND;
-  const int dim = rr_dim<D>(desc ? s.lvl : s.pd - 1);
-  const float nc = cukd::detail::pick<D>(p, dim);
-  const float qc = cukd::detail::pick<D>(q, dim);
-  if (desc) {
-    visits++;
-    s.cull = res.processCandidate(s.curr, cukd::detail::sqr_dist<D>(p, q));
-  }
-  const float diff = qc - nc;
-  const bool near = diff * diff < s.cull;
-  bool pop;
-  if (desc) {
-    const bool left_close = qc < nc;
-    const int l = 2 * s.curr + 1;
-    const int far = left_close ? l + 1 : l;
-    if (near && far < n) s.pending |= 2u << s.lvl;
-    s.curr = left_close ? l : l + 1;
-    s.off = 2u * s.off + (left_close ? stride : 2u * stride);
-    s.lvl++;
-    pop = s.curr >= n;
-  } else {
-    pop = !near;
-    if (near) {
-      // the far child: sibling of the path's node at depth pd
-      const int f = (((s.curr + 1) >> (s.lvl - s.pd)) ^ 1) - 1;
-      s.off = 2u * s.off + ((f & 1) ? stride : 2u * stride);
-      s.curr = f;
-      s.lvl = s.pd;
-      s.mode = SB_DESCEND;
-    }
-  }
-  if (pop) {
-    if (!s.pending) {
-      s.mode = SB_DONE;
-      return;
-    }
-    const int d = 31 - __clz((int)s.pending);
-    s.pending &= ~(1u << d);
-    s.pd = d;
-    s.mode = SB_POP;
-    s.off = (unsigned)(((s.curr + 1) >> (s.lvl - d + 1)) - 1) * stride;
-  }
-}
-
-// lists for which large sorted batches run with fewer resident waves (FCP
-// and k = 1 touch fewer nodes per query and measured faster at full
-// occupancy)
-template <class R> struct FewWaves { enum { ok = 0 }; };
-template <int K> struct FewWaves<cukd::FixedCandidateList<K>> { enum { ok = K >= 4 }; };
-
-// result types whose per-lane state is registers only (trees with
-// round-robin split dims only)
-template <class R> struct DualLane { enum { ok = 0 }; };
-template <> struct DualLane<cukd::FCPResult> { enum { ok = 1 }; };
-template <int K> struct DualLane<cukd::FixedCandidateList<K>> { enum { ok = 1 }; };
-
-template <int D, class R, bool FOREST>
-__global__ __launch_bounds__(256) void k_query2(TreeView t, const float *queries, int nq,
-                                                float cutoff, int k, const int32_t *order,
-                                                int32_t *ids, float *dist2, float *ret,
-                                                ListArgs la, ForestQ fq,
-                                                unsigned long long *stats)
-{
-  // XCD-aware workgroup order as in k_query; workgroup lb covers queries
-  // [lb*2*nt, (lb+1)*2*nt), wave w of it the 128 from lb*2*nt + 128*w, and
-  // lane l of the wave the two at +l and +64+l
-  const int nb = (int)gridDim.x;
-  const int xcd = (int)blockIdx.x & 7, q8 = nb >> 3, r8 = nb & 7;
-  const int lb = xcd * q8 + (xcd < r8 ? xcd : r8) + ((int)blockIdx.x >> 3);
-  const int i0 = lb * 2 * (int)blockDim.x + ((int)threadIdx.x >> 6) * 128 + ((int)threadIdx.x & 63);
-  if (i0 >= nq) return;
-  const bool has_b = i0 + 64 < nq;
-  const int qa = order ? order[i0] : i0;
-  const int qb = has_b ? (order ? order[i0 + 64] : i0 + 64) : qa;
-  const unsigned stride = (unsigned)t.stride;
-  const uint8_t *base = t.base + t.point_offset;
-  unsigned tb_a = 0, tb_b = 0;  // byte offset of the slot's tree in the forest
-  int n_a = t.n, n_b = t.n;
-  if constexpr (FOREST) {
-    const int ta = fq.seg_tree[segment_of(fq.seg_off, fq.nseg, qa)];
-    const int tb = fq.seg_tree[segment_of(fq.seg_off, fq.nseg, qb)];
-    const int oa = fq.tree_off[ta], ob = fq.tree_off[tb];
-    tb_a = (unsigned)oa * stride;
-    tb_b = (unsigned)ob * stride;
-    n_a = fq.tree_off[ta + 1] - oa;
-    n_b = fq.tree_off[tb + 1] - ob;
-  }
-  float pqa[D], pqb[D];
-#pragma unroll
-  for (int d = 0; d < D; d++) {
-    pqa[d] = queries[(size_t)qa * D + d];
-    pqb[d] = queries[(size_t)qb * D + d];
-  }
-  typename ResultOps<R>::State sta, stb;
-  R &ra = ResultOps<R>::init(sta, cutoff, k, qa, la, LdsCol{});
-  R &rb = ResultOps<R>::init(stb, cutoff, k, qb, la, LdsCol{});
-  SbSlot sa{n_a > 0 ? SB_DESCEND : SB_DONE, 0, 0, 0, 0u, 0u, ra.initialCullDist2()};
-  SbSlot sb{(has_b && n_b > 0) ? SB_DESCEND : SB_DONE, 0, 0, 0, 0u, 0u, rb.initialCullDist2()};
-  unsigned visits = 0;
-  while (sa.mode != SB_DONE || sb.mode != SB_DONE) {
-    // a finished query re-reads the other's node, so both loads stay in
-    // bounds and unconditional
-    unsigned oa = tb_a + sa.off, ob = tb_b + sb.off;
-    if (sa.mode == SB_DONE) oa = ob;
-    if (sb.mode == SB_DONE) ob = oa;
-    const float *src_a = (const float *)(base + oa);
-    const float *src_b = (const float *)(base + ob);
-    float pa[D], pb[D];
-#pragma unroll
-    for (int d = 0; d < D; d++) pa[d] = src_a[d];
-#pragma unroll
-    for (int d = 0; d < D; d++) pb[d] = src_b[d];
-    sb_step<D>(ra, pqa, pa, n_a, stride, sa, visits);
-    sb_step<D>(rb, pqb, pb, n_b, stride, sb, visits);
-  }
-  ResultOps<R>::write(sta, qa, k, ids, dist2, ret, la);
-  if (has_b) ResultOps<R>::write(stb, qb, k, ids, dist2, ret, la);
-  if (stats) atomicAdd(stats, (unsigned long long)visits);
-}
-
-// ---------------------------------------------------------------------------
-// two queries per lane, pending plane distances kept in LDS
-// ---------------------------------------------------------------------------
-// The traversal above re-reads a far child's parent on pop to recompute its
-// plane distance, which costs a loop iteration of its own. Here the plane
-// distance is stored when the far child is pushed (one LDS word per depth,
-// per query), so a pop is decided before the iteration's loads: a pop
-// that passes the cull test descends into the far child in the same
-// iteration, and only a pop that fails takes one. The visits, candidate
-// updates and visit counts are exactly those of the traversal above
-// (traverse-default-stack-based.h:58-107): the stored value is the same
-// diff*diff of the same node and query, tested against the same current
-// cull.
-struct SdSlot {
-  int mode;          // SB_DESCEND, SB_POP or SB_DONE
-  int curr;          // descend: node to visit; pop: end of the path (>= n)
-  int lvl;           // level of curr
-  unsigned off;      // descend: byte offset of curr
-  unsigned pending;  // bit d: the far child at depth d of the path is still to be visited
-  float topd;        // plane distance of the deepest pending far child
-  float cull;
-};
-
-// rows of per-query LDS words the traversal needs: a far child at depth d
-// exists only if 2^d <= n, and depth d is stored in row d - 1
-__host__ __device__ inline int sd_rows(int n)
-{
-  int r = 0;
-  while (r < 31 && (2ll << r) <= (long long)n) r++;
-  return r > 0 ? r : 1;
-}
-
-// pop the deepest pending far child: descend into it if its stored plane
-// distance is still below the cull, and reload the next stored distance
-__device__ inline void sd_pop(SdSlot &s, const float *col, int row_stride, unsigned stride)
-{
-  if (s.mode != SB_POP) return;
-  const int d = 31 - __clz((int)s.pending);
-  s.pending &= ~(1u << d);
-  if (s.topd < s.cull) {
-    const int f = (((s.curr + 1) >> (s.lvl - d)) ^ 1) - 1;
-    s.curr = f;
-    s.lvl = d;
-    s.off = (unsigned)f * stride;
-    s.mode = SB_DESCEND;
-  } else if (!s.pending) {
-    s.mode = SB_DONE;
-  }
-  if (s.pending) s.topd = col[(30 - __clz((int)s.pending)) * row_stride];
-}
-
-// visit curr, push its far child (with its plane distance) if it may hold
-// closer points, and step to the close child
-template <int D, class R>
-__device__ inline void sd_visit(R &res, const float (&q)[D], const float (&p)[D], int n,
-                                unsigned stride, SdSlot &s, float *col, int row_stride,
-                                unsigned &visits)
-{
-  if (s.mode != SB_DESCEND) return;
-  visits++;
-  s.cull = res.processCandidate(s.curr, cukd::detail::sqr_dist<D>(p, q));
-  const int dim = rr_dim<D>(s.lvl);
-  const float nc = cukd::detail::pick<D>(p, dim);
-  const float qc = cukd::detail::pick<D>(q, dim);
-  const float diff = qc - nc;
-  const float dd = diff * diff;
-  const bool left_close = qc < nc;
-  const int l = 2 * s.curr + 1;
-  const int far = left_close ? l + 1 : l;
-  if (dd < s.cull && far < n) {
-    s.pending |= 2u << s.lvl;
-    col[s.lvl * row_stride] = dd;
-    s.topd = dd;
-  }
-  s.curr = left_close ? l : l + 1;
-  s.off = 2u * s.off + (left_close ? stride : 2u * stride);
-  s.lvl++;
-  if (s.curr >= n) s.mode = s.pending ? SB_POP : SB_DONE;
-}
-
-// Dynamic LDS: sd_rows(n) rows of 2 * blockDim.x floats (row r holds depth
-// r + 1 of every slot of the workgroup; each lane only touches its own two
-// columns, so no barrier is needed).
-template <int D, class R, bool FOREST>
-__global__ __launch_bounds__(256) void k_query2s(TreeView t, const float *queries, int nq,
-                                                 float cutoff, int k, const int32_t *order,
-                                                 int32_t *ids, float *dist2, float *ret,
-                                                 ListArgs la, ForestQ fq,
-                                                 unsigned long long *stats)
-{
-  HIP_DYNAMIC_SHARED(float, s_pd);
-  const int nb = (int)gridDim.x;
-  const int xcd = (int)blockIdx.x & 7, q8 = nb >> 3, r8 = nb & 7;
-  const int lb = xcd * q8 + (xcd < r8 ? xcd : r8) + ((int)blockIdx.x >> 3);
-  const int i0 = lb * 2 * (int)blockDim.x + ((int)threadIdx.x >> 6) * 128 + ((int)threadIdx.x & 63);
-  if (i0 >= nq) return;
-  const bool has_b = i0 + 64 < nq;
-  const int qa = order ? order[i0] : i0;
-  const int qb = has_b ? (order ? order[i0 + 64] : i0 + 64) : qa;
-  const unsigned stride = (unsigned)t.stride;
-  const uint8_t *base = t.base + t.point_offset;
-  unsigned tb_a = 0, tb_b = 0;  // byte offset of the slot's tree in the forest
-  int n_a = t.n, n_b = t.n;
-  if constexpr (FOREST) {
-    const int ta = fq.seg_tree[segment_of(fq.seg_off, fq.nseg, qa)];
-    const int tb = fq.seg_tree[segment_of(fq.seg_off, fq.nseg, qb)];
-    const int oa = fq.tree_off[ta], ob = fq.tree_off[tb];
-    tb_a = (unsigned)oa * stride;
-    tb_b = (unsigned)ob * stride;
-    n_a = fq.tree_off[ta + 1] - oa;
-    n_b = fq.tree_off[tb + 1] - ob;
-  }
-  const int row_stride = 2 * (int)blockDim.x;
-  float *col_a = s_pd + threadIdx.x;
-  float *col_b = s_pd + blockDim.x + threadIdx.x;
-  float pqa[D], pqb[D];
-#pragma unroll
-  for (int d = 0; d < D; d++) {
-    pqa[d] = queries[(size_t)qa * D + d];
-    pqb[d] = queries[(size_t)qb * D + d];
-  }
-  typename ResultOps<R>::State sta, stb;
-  R &ra = ResultOps<R>::init(sta, cutoff, k, qa, la, LdsCol{});
-  R &rb = ResultOps<R>::init(stb, cutoff, k, qb, la, LdsCol{});
-  SdSlot sa{n_a > 0 ? SB_DESCEND : SB_DONE, 0, 0, 0u, 0u, 0.f, ra.initialCullDist2()};
-  SdSlot sb{(has_b && n_b > 0) ? SB_DESCEND : SB_DONE, 0, 0, 0u, 0u, 0.f, rb.initialCullDist2()};
-  unsigned visits = 0;
-  while (sa.mode != SB_DONE || sb.mode != SB_DONE) {
-    sd_pop(sa, col_a, row_stride, stride);
-    sd_pop(sb, col_b, row_stride, stride);
-    // a slot that does not descend this iteration re-reads the other's
-    // node (or the root), so both loads stay in bounds and unconditional
-    const bool da = sa.mode == SB_DESCEND, db = sb.mode == SB_DESCEND;
-    const unsigned oa = da ? tb_a + sa.off : (db ? tb_b + sb.off : 0u);
-    const unsigned ob = db ? tb_b + sb.off : oa;
-    const float *src_a = (const float *)(base + oa);
-    const float *src_b = (const float *)(base + ob);
-    float pa[D], pb[D];
-#pragma unroll
-    for (int d = 0; d < D; d++) pa[d] = src_a[d];
-#pragma unroll
-    for (int d = 0; d < D; d++) pb[d] = src_b[d];
-    sd_visit<D>(ra, pqa, pa, n_a, stride, sa, col_a, row_stride, visits);
-    sd_visit<D>(rb, pqb, pb, n_b, stride, sb, col_b, row_stride, visits);
-  }
-  ResultOps<R>::write(sta, qa, k, ids, dist2, ret, la);
-  if (has_b) ResultOps<R>::write(stb, qb, k, ids, dist2, ret, la);
-  if (stats) atomicAdd(stats, (unsigned long long)visits);
-}
+namespace cukd_amd {
 
 // ---------------------------------------------------------------------------
 // per-dimension launchers
@@ -692,72 +379,22 @@ struct QueryArgs {
   ListArgs la;
   ForestQ fq;
   unsigned long long *stats;
-  int block = 128;  // workgroup size: 64, 128 or 256
-  int lanes = 1;    // queries per lane: 1, or 2 (stack-based, register lists)
+  int block = 0;    // workgroup size: 64, 128 or 256 (0: the kernel's own default)
+  bool box = true;  // k_query_box where the call allows it
   uint64_t tree_bytes = 0;  // bytes of the tree array (forests: all trees)
-  int max_n = 0;            // forests: points of the largest tree (LDS rows of k_query2s)
+  int max_n = 0;            // forests: points of the largest tree
   bool presorted = false;   // queries already in Morton order (CUKD_QUERY_PRESORTED)
 };
 
 // persistent multi-round lists (cukd_knn_accumulate)
 enum { LIST_ACCUM = 100 };
 
-// gfx950 LDS per CU, and the batch size from which the two-query kernel
-// runs with fewer resident waves (a build option so that small test
-// batches can take that path too)
-#ifndef CUKD_QUERY2_FEW_WAVES_MIN_NQ
-#define CUKD_QUERY2_FEW_WAVES_MIN_NQ (1 << 19)
-#endif
-enum { LDS_PER_CU = 163840, QUERY2_FEW_WAVES_MIN_NQ = CUKD_QUERY2_FEW_WAVES_MIN_NQ };
+enum { LDS_PER_CU = 163840 };
 
 template <int D, int METHOD, class R>
 inline hipError_t launch_q(const QueryArgs &a, hipStream_t s)
 {
-  const int nt = a.block;
-  if constexpr (METHOD == CUKD_STACK_BASED && DualLane<R>::ok) {
-    if (a.lanes == 2 && a.t.dim_offset < 0) {
-      const int blocks = (a.nq + 2 * nt - 1) / (2 * nt);
-      // Large Morton-ordered batches run with fewer resident waves:
-      // workgroups are handed out in order (XCD-aware, along the Morton
-      // order), so fewer waves in flight means each XCD's active queries
-      // cover a smaller region and their nodes stay in its L2.  About 14
-      // waves per CU measured best for kNN-8 at 1M queries (10 % faster than
-      // 32, with 2.5x less L2-miss traffic); the dynamic LDS, unused by the
-      // kernel, only limits how many workgroups share a CU.
-      const bool few = FewWaves<R>::ok && (a.order || a.presorted) && nt == 128 &&
-                       a.nq >= QUERY2_FEW_WAVES_MIN_NQ;
-      const size_t lds = few ? LDS_PER_CU / 7 : 0;
-#ifndef CUKD_NO_STORED_PLANES
-      // Large batches, sorted or not, keep the pending plane distances in
-      // LDS.  The LDS rows for the deepest tree also bound the resident
-      // waves (6-7 workgroups per CU at 10M points), which suits unsorted
-      // batches too: fewer queries in flight thrash the L2s less.  A
-      // forest without a known largest tree keeps the kernel that re-reads
-      // parents.
-      if (nt == 128 && a.nq >= QUERY2_FEW_WAVES_MIN_NQ && (!a.fq.seg_off || a.max_n > 0)) {
-        const size_t need =
-            (size_t)sd_rows(a.fq.seg_off ? a.max_n : a.t.n) * 2 * nt * sizeof(float);
-        const size_t shm = need > lds ? need : lds;
-        if (a.fq.seg_off)
-          hipLaunchKernelGGL((k_query2s<D, R, true>), dim3(blocks), dim3(nt), shm, s, a.t,
-                             a.queries, a.nq, a.cutoff, a.k, a.order, a.ids, a.dist2, a.ret, a.la,
-                             a.fq, a.stats);
-        else
-          hipLaunchKernelGGL((k_query2s<D, R, false>), dim3(blocks), dim3(nt), shm, s, a.t,
-                             a.queries, a.nq, a.cutoff, a.k, a.order, a.ids, a.dist2, a.ret, a.la,
-                             a.fq, a.stats);
-        return hipGetLastError();
-      }
-#endif
-      if (a.fq.seg_off)
-        hipLaunchKernelGGL((k_query2<D, R, true>), dim3(blocks), dim3(nt), lds, s, a.t, a.queries,
-                           a.nq, a.cutoff, a.k, a.order, a.ids, a.dist2, a.ret, a.la, a.fq, a.stats);
-      else
-        hipLaunchKernelGGL((k_query2<D, R, false>), dim3(blocks), dim3(nt), lds, s, a.t, a.queries,
-                           a.nq, a.cutoff, a.k, a.order, a.ids, a.dist2, a.ret, a.la, a.fq, a.stats);
-      return hipGetLastError();
-    }
-  }
+  const int nt = a.block ? a.block : 128;
   const int blocks = (a.nq + nt - 1) / nt;
   // run-time-k lists: k words per lane of dynamic LDS (k <= 64 and nt <=
   // 256 keep it within one CU's 160 KiB)
@@ -769,9 +406,53 @@ inline hipError_t launch_q(const QueryArgs &a, hipStream_t s)
   return hipGetLastError();
 }
 
+template <int D, int METHOD, class L>
+inline hipError_t launch_box(const QueryArgs &a, hipStream_t s)
+{
+  const int nt = a.block ? a.block : 64;
+  const int rows = sd_rows(a.fq.seg_off ? a.max_n : a.t.n);
+  const size_t shm = (size_t)rows * nt * sizeof(float);
+  const int blocks = (a.nq + nt - 1) / nt;
+  hipLaunchKernelGGL((k_query_box<D, METHOD, L>), dim3(blocks), dim3(nt), shm, s, a.t, a.queries,
+                     a.nq, a.world_bounds, a.cutoff, a.eps, a.k, a.order, a.ids, a.dist2,
+                     a.ret, a.la, a.fq, rows);
+  return hipGetLastError();
+}
+
+// k_query_box serves trees with round-robin dims and 32-bit node offsets.
+// Counted traversals (cukd_set_traversal_stats) run k_query, whose visits
+// are the reference's, and so do NaN cutoffs, whose keys have no order as
+// doubles.
+inline bool box_ok(const QueryArgs &a)
+{
+  const uint64_t bytes = a.fq.seg_off ? a.tree_bytes : (uint64_t)a.t.n * (uint64_t)a.t.stride;
+  return a.box && !a.stats && a.t.dim_offset < 0 && bytes <= 0xffffffffull &&
+         a.cutoff == a.cutoff;
+}
+
 template <int D, int METHOD>
 inline hipError_t launch_method(const QueryArgs &a, hipStream_t s)
 {
+  if (box_ok(a)) {
+    if (a.list_kind < 0) return launch_box<D, METHOD, RegClosest>(a, s);
+    if (a.list_kind == CUKD_LIST_FIXED) {
+      if (a.k == 1) return launch_box<D, METHOD, RegSorted<1>>(a, s);
+      if (a.k <= 4) return launch_box<D, METHOD, RegSorted<4>>(a, s);
+      if (a.k <= 8) return launch_box<D, METHOD, RegSorted<8>>(a, s);
+      if (a.k <= 16) return launch_box<D, METHOD, RegSorted<16>>(a, s);
+      if (a.k <= 24) return launch_box<D, METHOD, RegSorted<24>>(a, s);
+      if (a.k <= 32) return launch_box<D, METHOD, RegSorted<32>>(a, s);
+      if (a.k <= 48) return launch_box<D, METHOD, RegSorted<48>>(a, s);
+      return launch_box<D, METHOD, RegSorted<64>>(a, s);
+    }
+    // heap lists, also the persistent ones of a multi-round query
+    if (a.k <= 8) return launch_box<D, METHOD, RegHeap<8>>(a, s);
+    if (a.k <= 16) return launch_box<D, METHOD, RegHeap<16>>(a, s);
+    if (a.k <= 24) return launch_box<D, METHOD, RegHeap<24>>(a, s);
+    if (a.k <= 32) return launch_box<D, METHOD, RegHeap<32>>(a, s);
+    if (a.k <= 48) return launch_box<D, METHOD, RegHeap<48>>(a, s);
+    return launch_box<D, METHOD, RegHeap<64>>(a, s);
+  }
   if (a.list_kind < 0) return launch_q<D, METHOD, cukd::FCPResult>(a, s);
   if (a.list_kind == CUKD_LIST_HEAP) return launch_q<D, METHOD, LdsHeapList>(a, s);
   if (a.list_kind == LIST_ACCUM) return launch_q<D, METHOD, AccumList>(a, s);

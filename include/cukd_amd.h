@@ -89,13 +89,13 @@ typedef struct cukd_mem_resource {
                              the fastest for later calls; results are the
                              same for every choice.  Not for multi-round
                              lists (they only use an already tuned choice) */
-#define CUKD_QUERY_ONE_PER_LANE 4 /* one query per lane everywhere.  By
-                             default the stack-based traversal with FCP or
-                             a FixedCandidateList of k = 1/4/8/16 over a
-                             tree with round-robin split dims (and under
-                             4 GiB) steps two queries per lane, so twice as
-                             many node loads are in flight; results are
-                             identical either way */
+#define CUKD_QUERY_ONE_PER_LANE 4 /* the traversals of cukd/traverse.h as
+                             they stand, node for node.  By default queries
+                             over a tree with round-robin split dims (and
+                             under 4 GiB) also skip subtrees whose cell is
+                             beyond the cull distance and keep their lists
+                             in registers; results are identical either
+                             way */
 #define CUKD_QUERY_PRESORTED 8 /* the queries are already in Morton order
                              (e.g. permuted by cukd_query_order): launch
                              with the shape of a CUKD_QUERY_SORT launch,
