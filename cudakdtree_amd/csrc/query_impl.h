@@ -484,6 +484,7 @@ struct SpatialBounds {
 struct SpatialArgs {
   const cukd_spatial_node *nodes;
   const uint32_t *prim_ids;
+  int num_nodes;
   TreeView data;
   SpatialBounds bounds;
   const float *queries;
@@ -491,11 +492,17 @@ struct SpatialArgs {
   float cutoff;
   int k;
   int list_kind;  // -1 = FCP
+  const int32_t *order;  // launch order (nullable)
+  bool prune;            // box pruning allowed
   int32_t *ids;
   float *dist2;
   float *ret;
   unsigned long long *stats;  // node + leaf-point visits (fcp.h:294,327), nullable
 };
+// bytes of points from which large spatial batches run in Morton order: an
+// L2's size
+constexpr uint64_t SPATIAL_ORDER_MIN_BYTES = (uint64_t)4 << 20;
+bool spatial_prunable(const cukd_spatial_tree *tree, int D);
 hipError_t launch_spatial_query(int D, int method, const SpatialArgs &a, hipStream_t s);
 int spatial_build_impl(cukd_spatial_tree *tree, const void *d_points, int n, const cukd_layout &L,
                        int leaf_threshold, hipStream_t s, const MemResource &mem);

@@ -18,7 +18,8 @@
 // reference does (spatial-kdtree.h:545-567).
 //
 // Queries: stack-based and closest-corner traversal with the reference's
-// 50-entry stack and overflow behaviour (fcp.h:256-427, knn.h:566-752).
+// results, its 50-entry stack's overflow included (fcp.h:256-427,
+// knn.h:566-752).
 #pragma clang fp contract(off)
 #include <new>
 
@@ -149,9 +150,11 @@ void scan_exclusive(const uint32_t *in, uint32_t *out, long long n, uint32_t *sc
 // ---------------------------------------------------------------------------
 // build kernels
 // ---------------------------------------------------------------------------
-__global__ void k_sp_init(SpNode *nodes, uint32_t *pos_prim, uint32_t *pos_node, int n, int D)
+__global__ void k_sp_init(SpNode *nodes, uint32_t *pos_prim, uint32_t *pos_node, uint32_t *degen,
+                          int n, int D)
 {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i == 0) *degen = 0u;
   if (i < 2) {
     SpNode &t = nodes[i];
     for (int d = 0; d < D; d++) { t.lo[d] = abox_enc(3.402823466e+38f); t.hi[d] = abox_enc(-3.402823466e+38f); }
@@ -199,8 +202,8 @@ __global__ __launch_bounds__(256) void k_sp_root_bounds(SpNode *nodes, const uin
 }
 
 // selectSplits (spatial-kdtree.h:316-396) for the open nodes [a, b)
-__global__ void k_sp_decide(SpNode *nodes, uint32_t *split_flag, int a, int b, int D,
-                            uint32_t threshold)
+__global__ void k_sp_decide(SpNode *nodes, uint32_t *split_flag, uint32_t *degen, int a, int b,
+                            int D, uint32_t threshold)
 {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (a + i >= b) return;
@@ -226,7 +229,10 @@ __global__ void k_sp_decide(SpNode *nodes, uint32_t *split_flag, int a, int b, i
       pos = 0.5f * (lo + hi);
       if (pos == lo || pos == hi) widest = -1;
     }
-    if (widest < 0) pos = abox_dec(t.lo[0]);
+    if (widest < 0) {
+      pos = abox_dec(t.lo[0]);
+      *degen = 1u;  // same value from every writer
+    }
     t.dim = widest;
     t.pos = pos;
     t.state = SP_SPLIT;
@@ -419,6 +425,25 @@ __global__ void k_sp_bounds_out(const SpNode *nodes, uint32_t *bounds, int D, bo
   }
 }
 
+// The bounds' last two words, unused below 8 dims, record that queries may
+// prune by box (k_spatial_query): no degenerate split, and no path of 50
+// inner nodes.  A tree without the record is queried without.
+enum : int32_t { SP_MARK = 0x70727562, SP_MARK2 = 0x786f622e };
+static void spatial_set_prunable(cukd_spatial_tree *tree, int D, bool ok)
+{
+  if (D >= CUKD_MAX_DIMS || !ok) return;
+  tree->ibounds[2 * CUKD_MAX_DIMS - 2] = SP_MARK;
+  tree->ibounds[2 * CUKD_MAX_DIMS - 1] = SP_MARK2;
+}
+
+bool spatial_prunable(const cukd_spatial_tree *tree, int D)
+{
+  return D < CUKD_MAX_DIMS && tree->ibounds[2 * CUKD_MAX_DIMS - 2] == SP_MARK &&
+         tree->ibounds[2 * CUKD_MAX_DIMS - 1] == SP_MARK2;
+}
+
+enum { SP_DEPTH = 50 };  // the reference's traversal stack (fcp.h:265)
+
 int spatial_build_impl(cukd_spatial_tree *tree, const void *d_points, int n, const cukd_layout &L,
                        int leaf_threshold, hipStream_t s, const MemResource &mem)
 {
@@ -443,14 +468,15 @@ int spatial_build_impl(cukd_spatial_tree *tree, const void *d_points, int n, con
   uint32_t *pflag = (uint32_t *)(tmp + o_pflag), *pexcl = (uint32_t *)(tmp + o_pexcl);
   uint32_t *scratch = (uint32_t *)(tmp + o_scan);
   uint32_t *num_split = (uint32_t *)(tmp + o_misc);
-  uint32_t *bounds_dev = (uint32_t *)(tmp + o_misc + 64);
+  uint32_t *bounds_dev = (uint32_t *)(tmp + o_misc + 64);  // 2 * D words, then degen
+  uint32_t *degen = bounds_dev + 2 * D;
   const bool isf = L.scalar_type == CUKD_SCALAR_F32;
   const uint8_t *pts = (const uint8_t *)d_points;
   int rc = CUKD_OK;
   hipError_t e = hipSuccess;
 
   hipLaunchKernelGGL(k_sp_init, dim3((unsigned)((nn + 255) / 256)), dim3(256), 0, s, nodes, pp[0],
-                     pn[0], n, D);
+                     pn[0], degen, n, D);
   if (n > 0) {
     int blocks = (n + 255) / 256;
     if (blocks > 2048) blocks = 2048;
@@ -458,12 +484,14 @@ int spatial_build_impl(cukd_spatial_tree *tree, const void *d_points, int n, con
   }
   // open nodes [a, b); node 1 is the reference's reserved empty leaf, so
   // the first children are numbered from 2
-  int cur = 0, a = 0, b = 1, next = 2;
+  int cur = 0, a = 0, b = 1, next = 2, levels = 0;
   const int gp = (n + 255) / 256;
   while (a < b) {
+    levels++;
     const int cnt = b - a;
     const int g = (cnt + 255) / 256;
-    hipLaunchKernelGGL(k_sp_decide, dim3(g), dim3(256), 0, s, nodes, nflag, a, b, D, thr);
+    hipLaunchKernelGGL(k_sp_decide, dim3(g), dim3(256), 0, s, nodes, nflag, degen, a, b, D,
+                       thr);
     scan_exclusive(nflag, nexcl, cnt, scratch, s);
     hipLaunchKernelGGL(k_sp_alloc, dim3(g), dim3(256), 0, s, nodes, (const uint32_t *)nexcl, a, b, next,
                        D);
@@ -506,11 +534,12 @@ int spatial_build_impl(cukd_spatial_tree *tree, const void *d_points, int n, con
                          (const uint32_t *)nexcl, out_nodes, num_nodes, isf);
       hipLaunchKernelGGL(k_sp_bounds_out, dim3(1), dim3(64), 0, s, (const SpNode *)nodes,
                          bounds_dev, D, isf);
-      uint32_t hb[2 * CUKD_MAX_DIMS];
-      e = hipMemcpyAsync(hb, bounds_dev, 4 * 2 * D, hipMemcpyDeviceToHost, s);
+      uint32_t hb[2 * CUKD_MAX_DIMS + 1];
+      e = hipMemcpyAsync(hb, bounds_dev, 4 * (2 * D + 1), hipMemcpyDeviceToHost, s);
       if (e == hipSuccess) e = hipStreamSynchronize(s);
       if (e == hipSuccess) {
         for (int i = 0; i < 2 * CUKD_MAX_DIMS; i++) tree->ibounds[i] = i < 2 * D ? (int32_t)hb[i] : 0;
+        spatial_set_prunable(tree, D, levels <= SP_DEPTH && hb[2 * D] == 0u);
         tree->nodes = out_nodes;
         tree->prim_ids = out_prims;
         tree->data = d_points;
@@ -537,26 +566,216 @@ int spatial_build_impl(cukd_spatial_tree *tree, const void *d_points, int n, con
 // spatial queries
 // ---------------------------------------------------------------------------
 
-// The stack-based query with a register-resident result keeps the first
-// SP_STACK_COLS entries of its traversal stack in LDS columns: the stack
-// is indexed at run time, so a per-lane array lives in scratch.  The
-// 0.05-radius queries of the spatial config rarely go deeper.  (kNN-16 of
-// 2M queries over 4M float4 points: 15.9 -> 12.3 ms.)  A list already in
-// LDS keeps the whole stack in scratch: with both, the 32 KiB per
-// workgroup cost more occupancy than the stack gained (heap kNN-16
-// 14.5 -> 16.3 ms).
+// One query per lane, with the results of the reference's traversals
+// (fcp.h:256-427, knn.h:566-752; cukd/spatial-kdtree.h states them) bit for
+// bit.
+//
+// Each iteration of a wave pops, takes up to SP_STEPS steps down, and offers
+// SP_POINTS points of a leaf: ids and points are loaded together, the
+// distances that may be accepted are offered in order, one per trip and lane.
+// A chunk's missing points repeat its first (branches around single loads
+// cost more than the loads).
+//
+// Box pruning (prune), as in k_query_box: the stack-based traversal also skips
+// a far child whose cell is beyond the cull distance, which no list accepts
+// from.  The host allows it where the tree is known to have no degenerate
+// split, whose children may lie on either side of the plane, and to be
+// shallower than the reference's stack, so that no skipped subtree could have
+// overflowed it.  Otherwise, and while visits are counted, nothing is
+// skipped beyond the reference's own test.
+//
+// Bound by lane use (15 of 64 per vector instruction: lanes pop, step and read
+// leaves at different times) and by a line access per point.  kNN-16 within
+// 0.05, 2M queries over 4M float4: 12.2 -> 3.8 ms with the Morton order (2.2
+// ms of it the order, 1.7 ms the box); closest-corner 13.5 -> 3.8; heap 16
+// 14.5 -> 3.9; kNN-64 over 4M float3, 1M queries: 28.7 -> 6.9 ms.  One step
+// per iteration 3.9 ms; node, ids and points loaded an iteration ahead, one
+// round trip each, 5.2 ms.
+//
+// The stack is indexed at run time: its first COLS entries (a node with its
+// parent's split dim in the top bits, and the cell's squared distance per
+// dim) are LDS columns, only deeper ones a per-lane array in scratch.
+enum { SP_POINTS = 4, SP_STEPS = 3, SP_DIM_SHIFT = 29 };
+enum { SP_POP = 0, SP_NODE = 1, SP_PTS = 2 };
+// 10 KB a wave: at 7.5 KB kNN-16 loses 3 % to scratch, at 5 KB 20 %, at 15 KB
+// 40 % to the waves that no longer fit
+template <int D> constexpr int sp_cols() { return 40 / (D + 1) < 16 ? 40 / (D + 1) : 16; }
+
+template <int D, bool CCT, class L>
+__global__ __launch_bounds__(256) void k_spatial_query(const cukd_spatial_node *nodes,
+                                                       const uint32_t *prim_ids, TreeView data,
+                                                       SpatialBounds bounds, const float *queries,
+                                                       int nq, float cutoff, int k, bool prune,
+                                                       const int32_t *order, int32_t *ids,
+                                                       float *dist2, float *ret,
+                                                       unsigned long long *stats)
+{
+  constexpr int W = D + 1, COLS = sp_cols<D>();
+  HIP_DYNAMIC_SHARED(uint32_t, s_stack);
+  // XCD-aware workgroup order, as in k_query
+  const int nb = (int)gridDim.x;
+  const int xcd = (int)blockIdx.x & 7, q8 = nb >> 3, r8 = nb & 7;
+  const int lb = xcd * q8 + (xcd < r8 ? xcd : r8) + ((int)blockIdx.x >> 3);
+  const int i = lb * (int)blockDim.x + (int)threadIdx.x;
+  if (i >= nq) return;
+  const int qi = order ? order[i] : i;
+  uint32_t *col = s_stack + (threadIdx.x >> 6) * (COLS * W * 64) + (threadIdx.x & 63);
+  uint32_t deep[(SP_DEPTH - COLS) * W];  // entries COLS and up
+  float q[D], o[D];                      // o: squared distance to the current cell, per dim
+#pragma unroll
+  for (int d = 0; d < D; d++) q[d] = queries[(size_t)qi * D + d];
+  L list;
+  list.init(cutoff, k, nullptr, true, 0);
+  float cull = list.cull();
+  unsigned visits = 0;
+  int sp = 0, stage = SP_NODE;
+  bool done = false, ok = true;
+#pragma unroll
+  for (int d = 0; d < D; d++) {
+    o[d] = 0.f;
+    if (CCT) {
+      float v = q[d];
+      v = v < bounds.v[d] ? bounds.v[d] : v;
+      v = bounds.v[D + d] < v ? bounds.v[D + d] : v;
+      const float df = v - q[d];
+      o[d] = df * df;
+    }
+  }
+  if (CCT) {
+    float s = o[0];
+#pragma unroll
+    for (int d = 1; d < D; d++) s = s + o[d];
+    done = s > cull;
+  }
+  uint32_t li = 0, le = 0;  // points of the current leaf still to be offered
+  int node = 0;
+  while (!done) {
+    if (stage == SP_POP) {
+      if (sp == 0) {
+        done = true;
+      } else {
+        --sp;
+        uint32_t e[W];
+        if (sp < COLS) {
+#pragma unroll
+          for (int w = 0; w < W; w++) e[w] = col[(sp * W + w) * 64];
+        } else {
+#pragma unroll
+          for (int w = 0; w < W; w++) e[w] = deep[(sp - COLS) * W + w];
+        }
+        float c[D], s = 0.f;
+#pragma unroll
+        for (int d = 0; d < D; d++) {
+          c[d] = __uint_as_float(e[1 + d]);
+          s = d == 0 ? c[0] : s + c[d];
+        }
+        const float plane2 = cukd::detail::pick<D>(c, (int)(e[0] >> SP_DIM_SHIFT));
+        if (!((CCT ? s : plane2) >= cull) && !(!CCT && prune && s > cull)) {
+          node = (int)(e[0] & ((1u << SP_DIM_SHIFT) - 1u));
+#pragma unroll
+          for (int d = 0; d < D; d++) o[d] = c[d];
+          stage = SP_NODE;
+        }
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < SP_STEPS; u++) {
+      if (stage != SP_NODE || done) break;
+      visits++;
+      const cukd_spatial_node nd = nodes[node];
+      // an empty root leaf (no points) has count 0 and offset ~0u
+      if (nd.count || nd.offset == 0xffffffffu) {
+        li = nd.offset;
+        le = nd.offset + nd.count;
+        stage = nd.count ? SP_PTS : SP_POP;
+      } else {
+        const int dim = nd.dim;
+        const float qc = cukd::detail::pick<D>(q, dim);
+        const bool left_close = qc < nd.pos;
+        const float diff = qc - nd.pos;
+        const float plane2 = diff * diff;
+        const uint32_t far_c = nd.offset + (left_close ? 1u : 0u);
+        node = (int)(nd.offset + (left_close ? 0u : 1u));
+        uint32_t e[W];
+        float s = 0.f;
+        e[0] = far_c | (uint32_t)dim << SP_DIM_SHIFT;
+#pragma unroll
+        for (int d = 0; d < D; d++) {
+          const float v = d == dim ? plane2 : o[d];
+          e[1 + d] = __float_as_uint(v);
+          s = d == 0 ? v : s + v;
+        }
+        if (CCT ? s < cull : plane2 < cull && !(prune && s > cull)) {
+          if (sp < COLS) {
+#pragma unroll
+            for (int w = 0; w < W; w++) col[(sp * W + w) * 64] = e[w];
+          } else {
+#pragma unroll
+            for (int w = 0; w < W; w++) deep[(sp - COLS) * W + w] = e[w];
+          }
+          if (++sp >= SP_DEPTH) {
+            ok = false;
+            done = true;
+          }
+        }
+      }
+    }
+    if (stage == SP_PTS && !done) {
+      const uint32_t m = le - li < SP_POINTS ? le - li : SP_POINTS;
+      visits += m;
+      uint32_t prim[SP_POINTS];
+      float p[SP_POINTS][D], d2[SP_POINTS];
+#pragma unroll
+      for (int j = 0; j < SP_POINTS; j++)
+        prim[j] = prim_ids[li + ((uint32_t)j < m ? j : 0)];
+#pragma unroll
+      for (int j = 0; j < SP_POINTS; j++) data.template point<D>((int)prim[j], p[j]);
+      unsigned in = 0;  // bit j: point j may be accepted
+#pragma unroll
+      for (int j = 0; j < SP_POINTS; j++) {
+        d2[j] = cukd::detail::sqr_dist<D>(p[j], q);
+        if ((uint32_t)j < m && d2[j] <= cull) in |= 1u << j;
+      }
+      // in order, one per trip and lane: most lanes take none or one
+      while (in) {
+        float v = d2[0];
+        uint32_t id = prim[0];
+        const unsigned low = in & (0u - in);
+#pragma unroll
+        for (int j = 1; j < SP_POINTS; j++) {
+          v = low == 1u << j ? d2[j] : v;
+          id = low == 1u << j ? prim[j] : id;
+        }
+        list.offer((int)id, v, cull);
+        in &= in - 1;
+      }
+      li += m;
+      if (li == le) stage = SP_POP;
+    }
+  }
+  if (stats) atomicAdd(stats, (unsigned long long)visits);
+  const size_t out = (size_t)qi * k;
+  list.write(k, ids + out, dist2 ? dist2 + out : nullptr, ret ? ret + qi : nullptr, nullptr);
+  // stack overflow: fcp reports no result, knn returns -1 (fcp.h:317-320,
+  // knn.h:620-623 print "STACK OVERFLOW" and return -1)
+  if (!ok) {
+    if (ret) ret[qi] = -1.f;
+    else ids[qi] = -1;
+  }
+}
+
+// The traversals of cukd/spatial-kdtree.h as they stand, with lists whose
+// keys are compared as integers: for NaN cutoffs, whose keys have no order
+// as doubles, for trees of 2^29 nodes and more, and for the closest point of
+// many queries in a small tree, where reading single points wins (1M queries
+// over 100K float4: 338 us here, 395 us above).  The first 16 entries of the
+// stack-based FCP's stack are LDS columns.
 template <bool CCT, class R> struct SpStackCols {
   enum { value = (CCT || ResultOps<R>::kLds) ? 0 : 16 };
 };
 
-template <bool CCT, class R>
-__host__ __device__ constexpr size_t sp_query_lds_words(int k, int nt)
-{
-  return (ResultOps<R>::kLds ? (size_t)k * 2 * nt : 0) + (size_t)SpStackCols<CCT, R>::value * 2 * nt;
-}
-
 template <int D, bool CCT, class R>
-__global__ __launch_bounds__(128) void k_spatial_query(const cukd_spatial_node *nodes,
+__global__ __launch_bounds__(128) void k_spatial_query_any(const cukd_spatial_node *nodes,
                                                        const uint32_t *prim_ids, TreeView data,
                                                        SpatialBounds bounds, const float *queries,
                                                        int nq, float cutoff, int k,
@@ -595,24 +814,51 @@ __global__ __launch_bounds__(128) void k_spatial_query(const cukd_spatial_node *
   }
 }
 
+template <int D, bool CCT, class L>
+static void launch_spatial_l(const SpatialArgs &a, hipStream_t s)
+{
+  const int nt = 64, blocks = (a.nq + nt - 1) / nt;
+  const size_t shm = (size_t)(D + 1) * sp_cols<D>() * nt * 4;
+  hipLaunchKernelGGL((k_spatial_query<D, CCT, L>), dim3(blocks), dim3(nt), shm, s, a.nodes,
+                     a.prim_ids, a.data, a.bounds, a.queries, a.nq, a.cutoff, a.k, a.prune, a.order, a.ids,
+                     a.dist2, a.ret, a.stats);
+}
+
 template <int D, bool CCT>
 static hipError_t launch_spatial_m(const SpatialArgs &a, hipStream_t s)
 {
-  const int nt = 128, blocks = (a.nq + nt - 1) / nt;
-  // dynamic LDS: k words per lane for run-time-k lists (64 KiB at k = 64),
-  // or the stack-based traversal's first 16 stack entries (16 KiB)
-#define CUKD_SPQ(R)                                                                          \
-  hipLaunchKernelGGL((k_spatial_query<D, CCT, R>), dim3(blocks), dim3(nt),                  \
-                     (sp_query_lds_words<CCT, R>(a.k, nt) * sizeof(uint32_t)), s, a.nodes,  \
-                     a.prim_ids, a.data, a.bounds, a.queries, a.nq, a.cutoff, a.k, a.ids,   \
-                     a.dist2, a.ret, a.stats)
-  if (a.list_kind < 0) CUKD_SPQ(cukd::FCPResult);
-  else if (a.list_kind == CUKD_LIST_HEAP) CUKD_SPQ(LdsHeapList);
-  else if (a.k == 4) CUKD_SPQ(cukd::FixedCandidateList<4>);
-  else if (a.k == 8) CUKD_SPQ(cukd::FixedCandidateList<8>);
-  else if (a.k == 16) CUKD_SPQ(cukd::FixedCandidateList<16>);
-  else CUKD_SPQ(DynFixedList);
+  const bool small_fcp = !CCT && a.list_kind < 0 && a.nq >= (1 << 19) &&
+                         (uint64_t)a.data.n * (uint64_t)a.data.stride < SPATIAL_ORDER_MIN_BYTES;
+  if (a.cutoff != a.cutoff || a.num_nodes > (1 << SP_DIM_SHIFT) || small_fcp) {
+    const int nt = 128, blocks = (a.nq + nt - 1) / nt;
+    // dynamic LDS: k 64-bit words per lane (64 KiB at k = 64), or the stack
+    // columns (16 KiB)
+#define CUKD_SPQ(R)                                                                             \
+  hipLaunchKernelGGL((k_spatial_query_any<D, CCT, R>), dim3(blocks), dim3(nt),                  \
+                     ((ResultOps<R>::kLds ? (size_t)a.k : (size_t)SpStackCols<CCT, R>::value) * \
+                      8 * nt),                                                                  \
+                     s, a.nodes, a.prim_ids,                                                    \
+                     a.data, a.bounds, a.queries, a.nq, a.cutoff, a.k, a.ids, a.dist2, a.ret,   \
+                     a.stats)
+    if (a.list_kind < 0) CUKD_SPQ(cukd::FCPResult);
+    else if (a.list_kind == CUKD_LIST_HEAP) CUKD_SPQ(LdsHeapList);
+    else CUKD_SPQ(DynFixedList);
 #undef CUKD_SPQ
+    return hipGetLastError();
+  }
+  if (a.list_kind < 0) launch_spatial_l<D, CCT, RegClosest>(a, s);
+  else if (a.list_kind == CUKD_LIST_FIXED) {
+    if (a.k <= 4) launch_spatial_l<D, CCT, RegSorted<4>>(a, s);
+    else if (a.k <= 8) launch_spatial_l<D, CCT, RegSorted<8>>(a, s);
+    else if (a.k <= 16) launch_spatial_l<D, CCT, RegSorted<16>>(a, s);
+    else if (a.k <= 32) launch_spatial_l<D, CCT, RegSorted<32>>(a, s);
+    else launch_spatial_l<D, CCT, RegSorted<64>>(a, s);
+  } else {
+    if (a.k <= 8) launch_spatial_l<D, CCT, RegHeap<8>>(a, s);
+    else if (a.k <= 16) launch_spatial_l<D, CCT, RegHeap<16>>(a, s);
+    else if (a.k <= 32) launch_spatial_l<D, CCT, RegHeap<32>>(a, s);
+    else launch_spatial_l<D, CCT, RegHeap<64>>(a, s);
+  }
   return hipGetLastError();
 }
 

@@ -238,8 +238,8 @@ typedef struct cukd_spatial_node {
 } cukd_spatial_node;
 
 typedef struct cukd_spatial_tree {
-  union {                        /* lower[num_dims] then upper[num_dims] */
-    float bounds[2 * 8];
+  union {                        /* lower[num_dims] then upper[num_dims]; */
+    float bounds[2 * 8];         /* the words after them are the library's */
     int32_t ibounds[2 * 8];
   };
   cukd_spatial_node *nodes;      /* device, num_nodes entries            */
