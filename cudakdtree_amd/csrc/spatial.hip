@@ -1,7 +1,9 @@
 // spatial.hip -- spatial k-d tree build and queries for gfx950.
 //
-// Build (spatial-kdtree.h:496-612 in the reference), one round per tree
-// level over all open nodes at once:
+// Build (spatial-kdtree.h:496-612 in the reference): spatial_build.h splits
+// large nodes round by round and finishes small ones in LDS; the kernels here
+// build trees too deep for that, one round per tree level over all open
+// nodes at once.  Both give the same tree:
 //   decide   : leaf if count <= threshold, else split the widest centroid
 //              extent at its centre (ties pick the earlier dim; a centre
 //              equal to either end makes a degenerate "dim -1" split)
@@ -68,6 +70,9 @@ struct SpNode {
   uint32_t count;
   uint32_t start;    // first position of this node's prims
   uint32_t offset;   // first child (inner)
+  uint32_t lex;      // left points before this node's, and its own (spatial_build.h)
+  uint32_t lcount;
+  int32_t level;
   int32_t dim;
   float pos;
   int32_t state;
@@ -444,11 +449,46 @@ bool spatial_prunable(const cukd_spatial_tree *tree, int D)
 
 enum { SP_DEPTH = 50 };  // the reference's traversal stack (fcp.h:265)
 
+}  // namespace cukd_amd
+
+#include "spatial_build.h"
+
+namespace cukd_amd {
+
+static int spatial_build_rounds(cukd_spatial_tree *tree, const void *d_points, int n,
+                                const cukd_layout &L, uint32_t thr, hipStream_t s,
+                                const MemResource &mem);
+
 int spatial_build_impl(cukd_spatial_tree *tree, const void *d_points, int n, const cukd_layout &L,
                        int leaf_threshold, hipStream_t s, const MemResource &mem)
 {
-  const int D = L.num_dims;
   const uint32_t thr = leaf_threshold <= 0 ? 8u : (uint32_t)leaf_threshold;
+  if (n > 0) {
+    const uint8_t *pts = (const uint8_t *)d_points;
+    bool deep = false;
+    int rc;
+    switch (L.num_dims) {
+      case 1: rc = spatial_build_items<1>(tree, pts, n, L, thr, s, mem, &deep); break;
+      case 2: rc = spatial_build_items<2>(tree, pts, n, L, thr, s, mem, &deep); break;
+      case 3: rc = spatial_build_items<3>(tree, pts, n, L, thr, s, mem, &deep); break;
+      case 4: rc = spatial_build_items<4>(tree, pts, n, L, thr, s, mem, &deep); break;
+      case 5: rc = spatial_build_items<5>(tree, pts, n, L, thr, s, mem, &deep); break;
+      case 6: rc = spatial_build_items<6>(tree, pts, n, L, thr, s, mem, &deep); break;
+      case 7: rc = spatial_build_items<7>(tree, pts, n, L, thr, s, mem, &deep); break;
+      default: rc = spatial_build_items<8>(tree, pts, n, L, thr, s, mem, &deep); break;
+    }
+    if (rc != CUKD_OK || !deep) return rc;
+  }
+  return spatial_build_rounds(tree, d_points, n, L, thr, s, mem);
+}
+
+// Round by round over all open nodes: trees of more than SPB_LEVELS levels,
+// and the empty one.
+static int spatial_build_rounds(cukd_spatial_tree *tree, const void *d_points, int n,
+                                const cukd_layout &L, uint32_t thr, hipStream_t s,
+                                const MemResource &mem)
+{
+  const int D = L.num_dims;
   const size_t max_nodes = 2 * (size_t)(n > 0 ? n : 1) + 2;
   const size_t nn = (size_t)(n > 0 ? n : 1);
   const size_t scan_words = scan_scratch_words((long long)(max_nodes > nn ? max_nodes : nn));
