@@ -54,7 +54,7 @@ EXPORTED_SYMBOLS = (
     "cukd_forest_destroy", "cukd_forest_fcp", "cukd_forest_knn", "cukd_forest_reserve_queries",
     "cukd_server_create", "cukd_server_submit", "cukd_server_poll",
     "cukd_server_get_stats", "cukd_server_destroy",
-    "cukd_last_error", "cukd_version",
+    "cukd_release_memory", "cukd_last_error", "cukd_version",
 )
 
 
@@ -182,6 +182,7 @@ def lib():
     L.cukd_server_get_stats.argtypes = [P, ctypes.POINTER(ServerStats)]
     L.cukd_server_destroy.argtypes = [P]
     L.cukd_set_traversal_stats.argtypes = [P]
+    L.cukd_release_memory.argtypes = []
     L.cukd_last_error.restype = ctypes.c_char_p
     L.cukd_last_error.argtypes = []
     L.cukd_version.restype = ctypes.c_int
@@ -527,6 +528,11 @@ class Forest:
             self.close()
         except Exception:
             pass
+
+
+def release_memory():
+    """Gives back the device memory the library keeps between calls."""
+    _check(lib().cukd_release_memory())
 
 
 def set_traversal_stats(counter):

@@ -410,6 +410,12 @@ int cukd_server_destroy(cukd_server *server);
  * as at traverse-default-stack-based.h:64) to *d_counter.  NULL disables. */
 int cukd_set_traversal_stats(unsigned long long *d_counter);
 
+/* Gives back the freed device memory that the library keeps for its next
+ * temporaries (up to 1 GiB per device, calls without a memory resource).
+ * Memory still in use, or freed on a stream that has not got there yet,
+ * stays. */
+int cukd_release_memory(void);
+
 /* Message of the last failed call on this thread ("" if none). */
 const char *cukd_last_error(void);
 
