@@ -8,11 +8,16 @@
 // ordering.  Order inside a cell is whatever the atomics give; it affects
 // speed, never results.
 //
-// A counting sort without returning global atomics: each tile of
-// QO_TILE queries counts its cells in LDS (k_qcount), one thread per cell
-// turns the per-tile counts into per-tile starts and a cell total
+// A counting sort without returning global atomics: each tile of queries
+// counts its cells in LDS (k_qcount), one thread per cell turns the
+// per-tile counts into per-tile starts, up to the cells of earlier blocks
 // (k_qcolscan), and each tile then places its queries from its starts with
-// LDS atomics (k_qplace), after scanning the cell totals itself.
+// LDS atomics (k_qplace).
+//
+// Bound by latency: a few LDS and memory rounds per kernel.  1M float3 queries:
+// 78 -> 63 us, 250K: 66 -> 45 us, where every workgroup had read the cell totals
+// at a stride of 128 bytes to scan them itself, into LDS columns of one
+// bank, and 16K-query tiles left most CUs idle.
 #include "cukd_common.h"
 
 namespace cukd_amd {
@@ -20,20 +25,12 @@ namespace cukd_amd {
 // 15-bit cells: on a 10M-point tree, kNN-8 over 1M uniform queries took
 // 0.789 / 0.764 / 0.747 / 0.737 ms launched in 9 / 12 / 15 / 18-bit cell
 // order; 2^15 counters (128 KB) are the most one workgroup's LDS holds.
-enum { MORTON_BITS = 15, QB_SLOTS = 32, QB_NT = 256 };
-enum { QO_CELLS = 1 << MORTON_BITS, QO_NT = 1024, QO_ITEMS = 16, QO_TILE = QO_NT * QO_ITEMS };
+enum { MORTON_BITS = 15, QB_NT = 256, QB_BLOCKS = 512 };
+enum { QO_CELLS = 1 << MORTON_BITS, QO_NT = 1024, QO_SCAN_NT = 256, QO_BLOCKS = QO_CELLS / QO_SCAN_NT };
 
-// Bounds accumulators: QB_SLOTS copies of (lo[CUKD_MAX_DIMS], hi[CUKD_MAX_DIMS])
-// as ordered keys; workgroup b folds into copy b % QB_SLOTS, so each word
-// takes few atomics, and readers fold the copies.
-enum { QB_WORDS = QB_SLOTS * 2 * CUKD_MAX_DIMS };
-
-// sets the accumulators to empty bounds
-__global__ void k_qinit(uint32_t *acc)
-{
-  for (int i = threadIdx.x; i < QB_WORDS; i += blockDim.x)
-    acc[i] = (i % (2 * CUKD_MAX_DIMS)) < CUKD_MAX_DIMS ? 0xffffffffu : 0u;
-}
+// Bounds: (lo[CUKD_MAX_DIMS], hi[CUKD_MAX_DIMS]) as ordered keys per workgroup
+// of k_qbounds, folded by their readers.
+enum { QB_WORDS = QB_BLOCKS * 2 * CUKD_MAX_DIMS };
 
 // Per-dim min / max of the nq*D query coordinates.  The flat array is read
 // coalesced with a thread stride T that is a multiple of D, so each thread
@@ -70,31 +67,35 @@ __global__ __launch_bounds__(QB_NT) void k_qbounds(uint32_t *acc, const float *q
     }
   }
   __syncthreads();
-  if ((int)threadIdx.x < D) {
-    uint32_t *a = acc + (blockIdx.x % QB_SLOTS) * 2 * CUKD_MAX_DIMS;
-    if (s_lo[threadIdx.x] != 0xffffffffu) atomicMin(&a[threadIdx.x], s_lo[threadIdx.x]);
-    if (s_hi[threadIdx.x] != 0u) atomicMax(&a[CUKD_MAX_DIMS + threadIdx.x], s_hi[threadIdx.x]);
+  if ((int)threadIdx.x < 2 * CUKD_MAX_DIMS) {
+    const int w = (int)threadIdx.x;
+    acc[blockIdx.x * 2 * CUKD_MAX_DIMS + w] =
+        w < CUKD_MAX_DIMS ? s_lo[w] : s_hi[w - CUKD_MAX_DIMS];
   }
 }
 
-// the batch box, folded from the accumulators (written by the previous
-// kernel, so plain loads see them): thread t < D folds lower bound t over
-// the QB_SLOTS copies, thread D + t upper bound t
-__device__ inline void qbox_load(const uint32_t *acc, int D, float *s_lo, float *s_hi)
+// the batch box, folded from the workgroups' bounds by a whole workgroup of
+// QO_NT threads; ends with a barrier
+__device__ inline void qbox_load(const uint32_t *acc, int nblocks, int D, float *s_lo, float *s_hi)
 {
-  const int t = (int)threadIdx.x;
-  if (t < 2 * D) {
-    const bool up = t >= D;
-    const int w0 = up ? CUKD_MAX_DIMS + (t - D) : t;
-    uint32_t v = up ? 0u : 0xffffffffu;
-#pragma unroll 8
-    for (int c = 0; c < QB_SLOTS; c++) {
-      const uint32_t x = acc[c * 2 * CUKD_MAX_DIMS + w0];
-      v = up ? max(v, x) : min(v, x);
-    }
-    const float f = __uint_as_float(unordered_key(v, true));
-    if (up) s_hi[t - D] = f;
-    else s_lo[t] = f;
+  __shared__ uint32_t s_key[2 * CUKD_MAX_DIMS];
+  const int tid = (int)threadIdx.x;
+  if (tid < 2 * CUKD_MAX_DIMS) s_key[tid] = tid < CUKD_MAX_DIMS ? 0xffffffffu : 0u;
+  __syncthreads();
+  // a thread's words are of one dim and side: QO_NT is a multiple of the row
+  const int w = tid % (2 * CUKD_MAX_DIMS);
+  const bool up = w >= CUKD_MAX_DIMS;
+  uint32_t v = up ? 0u : 0xffffffffu;
+  for (int i = tid; i < nblocks * 2 * CUKD_MAX_DIMS; i += QO_NT) {
+    const uint32_t x = acc[i];
+    v = up ? max(v, x) : min(v, x);
+  }
+  if (up) atomicMax(&s_key[w], v);
+  else atomicMin(&s_key[w], v);
+  __syncthreads();
+  if (tid < D) {
+    s_lo[tid] = __uint_as_float(unordered_key(s_key[tid], true));
+    s_hi[tid] = __uint_as_float(unordered_key(s_key[CUKD_MAX_DIMS + tid], true));
   }
   __syncthreads();
 }
@@ -119,16 +120,16 @@ __device__ inline uint32_t morton_cell(const float *x, const float *lo_, const f
   return code & ((1u << MORTON_BITS) - 1);
 }
 
-// The cells of a thread's queries in one tile, QO_BATCH at a time: every
-// coordinate load of a batch is issued before any is used.
+// The cells of a thread's queries in one tile of ITEMS * QO_NT, QO_BATCH at a
+// time: every coordinate load of a batch is issued before any is used.
 enum { QO_BATCH = 4, QO_NONE = 0xffffffffu };
-template <int DC>
-__device__ inline void tile_cells(uint32_t (&cell)[QO_ITEMS], const float *q, int nq,
+template <int DC, int ITEMS>
+__device__ inline void tile_cells(uint32_t (&cell)[ITEMS], const float *q, int nq,
                                   const float *s_lo, const float *s_hi)
 {
-  const long long i0 = (long long)blockIdx.x * QO_TILE + threadIdx.x;
+  const long long i0 = (long long)blockIdx.x * (ITEMS * QO_NT) + threadIdx.x;
 #pragma unroll
-  for (int k0 = 0; k0 < QO_ITEMS; k0 += QO_BATCH) {
+  for (int k0 = 0; k0 < ITEMS; k0 += QO_BATCH) {
     float x[QO_BATCH][DC];
 #pragma unroll
     for (int k = 0; k < QO_BATCH; k++) {
@@ -144,102 +145,154 @@ __device__ inline void tile_cells(uint32_t (&cell)[QO_ITEMS], const float *q, in
   }
 }
 
-// Cell counts of one tile of QO_TILE queries: row 'tile' of th (tile-major,
-// QO_CELLS words a row).
-template <int DC>
+// Cell counts of one tile: row 'tile' of th (tile-major, QO_CELLS words a
+// row).
+template <int DC, int ITEMS>
 __global__ __launch_bounds__(QO_NT) void k_qcount(uint32_t *th, const float *q, int nq,
-                                                 const uint32_t *acc)
+                                                 const uint32_t *acc, int nblocks)
 {
   __shared__ uint32_t h[QO_CELLS];
   __shared__ float s_lo[CUKD_MAX_DIMS], s_hi[CUKD_MAX_DIMS];
   for (int c = threadIdx.x; c < QO_CELLS; c += QO_NT) h[c] = 0u;
-  qbox_load(acc, DC, s_lo, s_hi);  // ends with a barrier
-  uint32_t cell[QO_ITEMS];
-  tile_cells<DC>(cell, q, nq, s_lo, s_hi);
+  qbox_load(acc, nblocks, DC, s_lo, s_hi);  // ends with a barrier
+  uint32_t cell[ITEMS];
+  tile_cells<DC, ITEMS>(cell, q, nq, s_lo, s_hi);
 #pragma unroll
-  for (int k = 0; k < QO_ITEMS; k++)
+  for (int k = 0; k < ITEMS; k++)
     if (cell[k] != QO_NONE) atomicAdd(&h[cell[k]], 1u);
   __syncthreads();
   uint32_t *row = th + (size_t)blockIdx.x * QO_CELLS;
   for (int c = threadIdx.x; c < QO_CELLS; c += QO_NT) row[c] = h[c];
 }
 
-// One thread per cell: the counts of the tiles become each tile's start
-// inside the cell (exclusive, in tile order), and tot[cell] the cell's
-// size.  Eight tiles' counts are loaded before any is rewritten.
-__global__ void k_qcolscan(uint32_t *th, uint32_t *tot, int ntiles)
+// The counts of the tiles become each tile's start among the cells of this
+// workgroup (cell order, then tile order), and tot[block] the workgroup's
+// queries.  QO_SPLIT threads per cell, each with a run of the tiles, and eight
+// tiles' counts in flight: the kernel is a chain of loads.
+enum { QO_SPLIT = 4 };
+__global__ __launch_bounds__(QO_SCAN_NT * QO_SPLIT) void k_qcolscan(uint32_t *th, uint32_t *tot,
+                                                                    int ntiles)
 {
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= QO_CELLS) return;
-  uint32_t run = 0;
-  for (int t0 = 0; t0 < ntiles; t0 += 8) {
+  __shared__ uint32_t part[QO_SPLIT][QO_SCAN_NT], wsum[QO_SCAN_NT / 64];
+  const int cl = (int)threadIdx.x % QO_SCAN_NT, g = (int)threadIdx.x / QO_SCAN_NT;
+  const int c = blockIdx.x * QO_SCAN_NT + cl;
+  const int lane = cl & 63, w = cl >> 6;
+  const int per = (ntiles + QO_SPLIT - 1) / QO_SPLIT;
+  const int ta = g * per, tz = ta + per < ntiles ? ta + per : ntiles;
+  uint32_t sum = 0;
+  for (int t0 = ta; t0 < tz; t0 += 8) {
     uint32_t v[8];
 #pragma unroll
-    for (int j = 0; j < 8; j++)
-      v[j] = t0 + j < ntiles ? th[(size_t)(t0 + j) * QO_CELLS + c] : 0u;
+    for (int j = 0; j < 8; j++) v[j] = t0 + j < tz ? th[(size_t)(t0 + j) * QO_CELLS + c] : 0u;
 #pragma unroll
-    for (int j = 0; j < 8; j++) {
-      if (t0 + j < ntiles) th[(size_t)(t0 + j) * QO_CELLS + c] = run;
-      run += v[j];
-    }
+    for (int j = 0; j < 8; j++) sum += v[j];
   }
-  tot[c] = run;
-}
-
-// Places one tile's queries: the cell starts are the exclusive scan of the
-// cell totals plus the tile's start inside each cell; queries take
-// consecutive slots from there.
-template <int DC>
-__global__ __launch_bounds__(QO_NT) void k_qplace(int32_t *order, const uint32_t *th,
-                                                 const uint32_t *tot, const float *q, int nq,
-                                                 const uint32_t *acc)
-{
-  enum { CPT = QO_CELLS / QO_NT };  // cells per thread, consecutive
-  static_assert(QO_CELLS % QO_NT == 0, "cells per thread");
-  __shared__ uint32_t base[QO_CELLS];
-  __shared__ uint32_t wsum[QO_NT / 64];
-  __shared__ float s_lo[CUKD_MAX_DIMS], s_hi[CUKD_MAX_DIMS];
-  const int tid = (int)threadIdx.x, lane = tid & 63, w = tid >> 6;
-  uint32_t v[CPT], sum = 0;
+  part[g][cl] = sum;
+  __syncthreads();
+  uint32_t all = 0, before = 0;
 #pragma unroll
-  for (int j = 0; j < CPT; j++) {
-    v[j] = tot[tid * CPT + j];
-    sum += v[j];
+  for (int i = 0; i < QO_SPLIT; i++) {
+    all += part[i][cl];
+    if (i < g) before += part[i][cl];
   }
-  // exclusive scan of the per-thread sums over the workgroup
-  uint32_t incl = sum;
+  uint32_t incl = all;
 #pragma unroll
   for (int o = 1; o < 64; o <<= 1) {
     const uint32_t u = (uint32_t)__shfl_up((int)incl, o);
     if (lane >= o) incl += u;
   }
-  if (lane == 63) wsum[w] = incl;
+  if (g == 0 && lane == 63) wsum[w] = incl;
   __syncthreads();
-  uint32_t run = incl - sum;
+  uint32_t run = incl - all;
   for (int i = 0; i < w; i++) run += wsum[i];
-  const uint32_t *row = th + (size_t)blockIdx.x * QO_CELLS;
+  if (g == 0 && cl == QO_SCAN_NT - 1) tot[blockIdx.x] = run + all;
+  run += before;
+  for (int t0 = ta; t0 < tz; t0 += 8) {
+    uint32_t v[8];
 #pragma unroll
-  for (int j = 0; j < CPT; j++) {
-    base[tid * CPT + j] = run + row[tid * CPT + j];
-    run += v[j];
+    for (int j = 0; j < 8; j++) v[j] = t0 + j < tz ? th[(size_t)(t0 + j) * QO_CELLS + c] : 0u;
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+      if (t0 + j < tz) th[(size_t)(t0 + j) * QO_CELLS + c] = run;
+      run += v[j];
+    }
   }
-  qbox_load(acc, DC, s_lo, s_hi);  // ends with a barrier
-  uint32_t cell[QO_ITEMS];
-  tile_cells<DC>(cell, q, nq, s_lo, s_hi);
-  const long long i0 = (long long)blockIdx.x * QO_TILE + threadIdx.x;
+}
+
+// Places one tile's queries: consecutive slots from the tile's start in each
+// cell, behind the queries of the earlier blocks' cells.
+template <int DC, int ITEMS>
+__global__ __launch_bounds__(QO_NT) void k_qplace(int32_t *order, const uint32_t *th,
+                                                 const uint32_t *tot, const float *q, int nq,
+                                                 const uint32_t *acc, int nblocks)
+{
+  static_assert(QO_BLOCKS <= 2 * 64 && QO_CELLS % QO_NT == 0, "one wave scans the blocks");
+  __shared__ uint32_t base[QO_CELLS];
+  __shared__ uint32_t s_blk[QO_BLOCKS];
+  __shared__ float s_lo[CUKD_MAX_DIMS], s_hi[CUKD_MAX_DIMS];
+  const int tid = (int)threadIdx.x;
+  const uint32_t *row = th + (size_t)blockIdx.x * QO_CELLS;
+  uint32_t v[QO_CELLS / QO_NT];
 #pragma unroll
-  for (int k = 0; k < QO_ITEMS; k++)
+  for (int j = 0; j < QO_CELLS / QO_NT; j++) v[j] = row[j * QO_NT + tid];
+  if (tid < 64) {
+    const uint32_t a = 2 * tid < QO_BLOCKS ? tot[2 * tid] : 0u;
+    const uint32_t b = 2 * tid + 1 < QO_BLOCKS ? tot[2 * tid + 1] : 0u;
+    uint32_t incl = a + b;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const uint32_t u = (uint32_t)__shfl_up((int)incl, o);
+      if (tid >= o) incl += u;
+    }
+    if (2 * tid < QO_BLOCKS) s_blk[2 * tid] = incl - a - b;
+    if (2 * tid + 1 < QO_BLOCKS) s_blk[2 * tid + 1] = incl - b;
+  }
+  qbox_load(acc, nblocks, DC, s_lo, s_hi);  // ends with a barrier
+#pragma unroll
+  for (int j = 0; j < QO_CELLS / QO_NT; j++) {
+    const int c = j * QO_NT + tid;
+    base[c] = v[j] + s_blk[c / QO_SCAN_NT];
+  }
+  uint32_t cell[ITEMS];
+  tile_cells<DC, ITEMS>(cell, q, nq, s_lo, s_hi);
+  __syncthreads();
+  const long long i0 = (long long)blockIdx.x * (ITEMS * QO_NT) + threadIdx.x;
+#pragma unroll
+  for (int k = 0; k < ITEMS; k++)
     if (cell[k] != QO_NONE) order[atomicAdd(&base[cell[k]], 1u)] = (int32_t)(i0 + (long long)k * QO_NT);
 }
 
 static size_t align256(size_t b) { return (b + 255) / 256 * 256; }
 
-static int order_tiles(int nq) { return (nq + QO_TILE - 1) / QO_TILE; }
+// queries per thread of a tile: the tiles of a small batch are small, so that
+// they spread over the CUs (each reads and writes 128 KB of counts, so no
+// smaller)
+static int order_items(int nq) { return nq <= (1 << 18) ? 4 : nq <= (1 << 20) ? 8 : 16; }
+static int order_tiles(int nq)
+{
+  const int tile = order_items(nq) * QO_NT;
+  return (nq + tile - 1) / tile;
+}
 
 size_t query_order_temp_bytes(int nq)
 {
-  return align256((size_t)nq * 4) + align256((size_t)order_tiles(nq) * QO_CELLS * 4) +
-         align256((size_t)QO_CELLS * 4) + QB_WORDS * 4 + 256;
+  // the tile size steps up with nq, so a smaller batch may have more tiles
+  int tiles = order_tiles(nq);
+  if (nq > (1 << 18)) tiles = tiles > order_tiles(1 << 18) ? tiles : order_tiles(1 << 18);
+  if (nq > (1 << 20)) tiles = tiles > order_tiles(1 << 20) ? tiles : order_tiles(1 << 20);
+  return align256((size_t)nq * 4) + align256((size_t)tiles * QO_CELLS * 4) +
+         align256((size_t)QO_BLOCKS * 4) + QB_WORDS * 4 + 256;
+}
+
+template <int DC, int ITEMS>
+static void launch_order(int32_t *order, uint32_t *th, uint32_t *tot, const uint32_t *acc,
+                         int nblocks, const float *q, int nq, int tiles, hipStream_t s)
+{
+  hipLaunchKernelGGL((k_qcount<DC, ITEMS>), dim3(tiles), dim3(QO_NT), 0, s, th, q, nq, acc, nblocks);
+  hipLaunchKernelGGL(k_qcolscan, dim3(QO_BLOCKS), dim3(QO_SCAN_NT * QO_SPLIT), 0, s, th, tot,
+                     tiles);
+  hipLaunchKernelGGL((k_qplace<DC, ITEMS>), dim3(tiles), dim3(QO_NT), 0, s, order,
+                     (const uint32_t *)th, (const uint32_t *)tot, q, nq, acc, nblocks);
 }
 
 // Writes the launch order of nq queries into the front of 'tmp' (which
@@ -249,30 +302,25 @@ int32_t *make_query_order(void *tmp, const float *q, int nq, int D, hipStream_t 
   uint8_t *t = (uint8_t *)tmp;
   int32_t *order = (int32_t *)t;
   if (nq <= 0) return order;
-  const int tiles = order_tiles(nq);
+  const int tiles = order_tiles(nq), items = order_items(nq);
   t += align256((size_t)nq * 4);
   uint32_t *th = (uint32_t *)t;
   t += align256((size_t)tiles * QO_CELLS * 4);
   uint32_t *tot = (uint32_t *)t;
-  t += align256((size_t)QO_CELLS * 4);
+  t += align256((size_t)QO_BLOCKS * 4);
   uint32_t *acc = (uint32_t *)t;
-  hipLaunchKernelGGL(k_qinit, dim3(1), dim3(256), 0, s, acc);
   const long long E = (long long)nq * D;
   long long blocks = (E + QB_NT * 4 - 1) / (QB_NT * 4);
-  if (blocks > 1024) blocks = 1024;
+  if (blocks > QB_BLOCKS) blocks = QB_BLOCKS;
   long long T = blocks * QB_NT;
   T -= T % D;
   if (T < D) T = D;  // E >= D, and blocks * QB_NT >= 256 >= D
   hipLaunchKernelGGL(k_qbounds, dim3((unsigned)blocks), dim3(QB_NT), 0, s, acc, q, E, D, T);
-#define CUKD_QORDER_CASE(DCv)                                                                  \
-  case DCv:                                                                                    \
-    hipLaunchKernelGGL(k_qcount<DCv>, dim3(tiles), dim3(QO_NT), 0, s, th, q, nq,              \
-                       (const uint32_t *)acc);                                                 \
-    hipLaunchKernelGGL(k_qcolscan, dim3((QO_CELLS + 255) / 256), dim3(256), 0, s, th, tot,    \
-                       tiles);                                                                 \
-    hipLaunchKernelGGL(k_qplace<DCv>, dim3(tiles), dim3(QO_NT), 0, s, order,                  \
-                       (const uint32_t *)th, (const uint32_t *)tot, q, nq,                     \
-                       (const uint32_t *)acc);                                                 \
+#define CUKD_QORDER_CASE(DCv)                                                                   \
+  case DCv:                                                                                     \
+    if (items == 4) launch_order<DCv, 4>(order, th, tot, acc, (int)blocks, q, nq, tiles, s);    \
+    else if (items == 8) launch_order<DCv, 8>(order, th, tot, acc, (int)blocks, q, nq, tiles, s); \
+    else launch_order<DCv, 16>(order, th, tot, acc, (int)blocks, q, nq, tiles, s);              \
     break
   switch (D) {
     CUKD_QORDER_CASE(1);
