@@ -268,7 +268,8 @@ __device__ inline void flush_hist(uint32_t *h, const uint32_t *s_h, int nbins)
 // histograms, cursors, tie bounds: zwords words from zero), which the
 // levels' first launches need zeroed.  (A fill kernel rather than
 // hipMemsetAsync, so that a forest build can be captured into a graph.)
-__global__ __launch_bounds__(256) void k_copy_in(TreeSet<InTree> set, uint8_t *data,
+enum { COPY_NT = 1024 };
+__global__ __launch_bounds__(COPY_NT) void k_copy_in(TreeSet<InTree> set, uint8_t *data,
                                                  uint32_t *idx, uint32_t *key,
                                                  const uint8_t *points, cukd_layout L,
                                                  const SegState *st, int explicit_dim,
@@ -1993,6 +1994,306 @@ __global__ __launch_bounds__(NT) void k_finish_rank(
 }
 
 // ---------------------------------------------------------------------------
+// one top level of subtrees that fit a workgroup: select, tie-break and
+// partition in one launch
+// ---------------------------------------------------------------------------
+// The launches above spread one subtree over many workgroups, so they meet
+// through memory at five kernel boundaries a level (about 45 us for a level
+// of 100K points, whatever its size).  A subtree of at most WG_MAX elements
+// is taken by one workgroup instead, with its keys in registers:
+//  * the range that holds the pivot's key shrinks by 2048 linear bins at a
+//    time until at most WG_CAND elements lie in it (one pass, nearly always;
+//    where more elements share one key, their next word takes over);
+//  * those few are ranked against each other by their whole keys, one lane
+//    each, which finds the pivot and settles ties;
+//  * the partition ranks by ballots in (item, wave, lane) order, as
+//    k_partition does.
+// The tree is the same: a level depends on the pivots only, not on the order
+// inside the children.
+// Bound by barriers and memory latency: 13 us for a level of 800-element
+// subtrees, 20 at 3K, 30 at 6K and 47 at 12.5K, where the five launches take
+// 42 .. 49 us; a level of 1024 subtrees of 9.8K (10M points) takes 100 us less.
+// Builds: 2000 points 159 -> 118 us, 10K 286 -> 193, 100K 462 -> 377.
+enum { WG_NT = 1024, WG_E = 16, WG_MAX = WG_NT * WG_E, WG_BINS = 2048, WG_CAND = 256 };
+
+//
+// SW: elements of at most SW words pass through registers (0: any size).
+template <bool EXPLICIT, int SW>
+__global__ __launch_bounds__(WG_NT) void k_level_wg(TreeSet<LvlTree> set, int level,
+                                                    const uint32_t *key, const uint8_t *data,
+                                                    const uint32_t *idx, SegState *st,
+                                                    uint8_t *ndata, uint32_t *nidx,
+                                                    uint32_t *nkey, uint8_t *out, cukd_layout L)
+{
+  enum { NW = WG_NT / 64 };
+  __shared__ uint32_t s_v[WG_MAX], s_hist[WG_BINS];
+  __shared__ uint32_t s_wsum[NW], s_lo[NW], s_hi[NW];
+  __shared__ uint32_t s_pick[3];  // bin, elements of the lower bins, elements of the bin
+  __shared__ uint32_t s_cval[WG_CAND], s_cpos[WG_CAND], s_ncand;
+  __shared__ uint32_t s_pw[MAX_WORDS];  // the pivot's words
+  __shared__ int s_pivot;               // its position
+  __shared__ uint32_t s_cnt[2 * WG_E * NW];
+  __shared__ uint8_t s_rank[WG_MAX];    // rank of an element among its wave's of one item and side
+  __shared__ uint32_t s_cdim[2];
+  __shared__ SegState s_st;
+  __shared__ LvlTree s_tree;
+  const int tid = (int)threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  if (tid == 0) {
+    s_tree = find_tree(set, (int)blockIdx.x, [](const LvlTree &x) { return x.hseg; });
+    s_ncand = 0u;
+  }
+  __syncthreads();
+  const LvlTree tr = s_tree;
+  const int s = (int)blockIdx.x - tr.hseg, D = L.num_dims;
+  LevelGeom g, gn;
+  g.init(tr.n, level);
+  gn.init(tr.n, level + 1);
+  const int m = g.size(s), node = (1 << level) - 1 + s;
+  const size_t at = (size_t)tr.base + g.offset(s);
+  key += at;
+  data += at * L.stride;
+  idx += at;
+  ndata += (size_t)tr.base * L.stride;
+  nidx += tr.base;
+  nkey += tr.base;
+  const bool isf = L.scalar_type == CUKD_SCALAR_F32;
+  // The values of the word being resolved, a thread's own at e * WG_NT + tid
+  // (in LDS: 16 registers more spill, and make the rare paths unrolled code).
+  uint32_t mask = 0;
+#pragma unroll 8
+  for (int e = 0; e < WG_E; e++) {
+    const int p = e * WG_NT + tid;
+    if (p >= m) continue;
+    s_v[p] = key[p];
+    mask |= 1u << e;
+  }
+  uint32_t chain = 0;
+  int clen = 0, dim = level % D;
+  if (EXPLICIT) {
+    if (tid == 0) s_st = st[tr.seg + s];
+    __syncthreads();
+    chain = s_st.chain;
+    clen = (int)s_st.chain_len;
+    dim = (int)s_st.dim;
+  } else {
+    for (int l = level; l >= 0 && clen < D; l--) chain |= (uint32_t)(l % D) << (4 * clen++);
+  }
+  // word w >= 1 of the key of the element at p: a coordinate, or the index
+  auto word = [&](int w, int p) {
+    return w < clen ? ordered_key(load_coord_bits(data + (size_t)p * L.stride, L,
+                                                  (int)chain_at(chain, w)), isf)
+                    : idx[p];
+  };
+  // the candidates: elements of 'mask' whose word w lies in [lo, hi]
+  uint32_t rem = (uint32_t)subtree_size(2 * node + 1, tr.n);  // the pivot's rank among them
+  uint32_t cnt = (uint32_t)m, lo = 0u, hi = 0u;
+  int w = 0;
+  for (;;) {
+    lo = 0xffffffffu;
+    hi = 0u;
+#pragma unroll 4
+    for (int e = 0; e < WG_E; e++) {
+      if (!((mask >> e) & 1u)) continue;
+      const uint32_t x = s_v[e * WG_NT + tid];
+      lo = min(lo, x);
+      hi = max(hi, x);
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+      lo = min(lo, (uint32_t)__shfl_xor((int)lo, o));
+      hi = max(hi, (uint32_t)__shfl_xor((int)hi, o));
+    }
+    if (lane == 0) {
+      s_lo[wave] = lo;
+      s_hi[wave] = hi;
+    }
+    __syncthreads();
+    for (int i = 0; i < NW; i++) {
+      lo = min(lo, s_lo[i]);
+      hi = max(hi, s_hi[i]);
+    }
+    while (cnt > (uint32_t)WG_CAND && lo < hi) {
+      const int bits = 32 - __clz((int)(hi - lo));
+      const int sh = bits > 11 ? bits - 11 : 0;
+      for (int i = tid; i < WG_BINS; i += WG_NT) s_hist[i] = 0u;
+      __syncthreads();
+#pragma unroll 4
+      for (int e = 0; e < WG_E; e++) {
+        if (!((mask >> e) & 1u)) continue;
+        const uint32_t x = s_v[e * WG_NT + tid];
+        if (x >= lo && x <= hi) atomicAdd(&s_hist[(x - lo) >> sh], 1u);
+      }
+      __syncthreads();
+      const uint32_t b0 = s_hist[2 * tid], b1 = s_hist[2 * tid + 1];
+      const uint32_t before = rk_block_scan<WG_NT>(b0 + b1, s_wsum);
+      if (rem >= before && rem < before + b0 + b1) {
+        const bool second = rem >= before + b0;
+        s_pick[0] = 2u * (uint32_t)tid + (second ? 1u : 0u);
+        s_pick[1] = second ? before + b0 : before;
+        s_pick[2] = second ? b1 : b0;
+      }
+      __syncthreads();
+      rem -= s_pick[1];
+      cnt = s_pick[2];
+      lo += s_pick[0] << sh;
+      const uint32_t width = (1u << sh) - 1u;
+      hi = hi - lo > width ? lo + width : hi;
+    }
+    if (cnt <= (uint32_t)WG_CAND) break;
+    // more elements share this word than can be ranked: their next word
+    // (the last one, the index, is each element's own)
+    w++;
+#pragma unroll 1
+    for (int e = 0; e < WG_E; e++) {
+      const int p = e * WG_NT + tid;
+      if (!((mask >> e) & 1u)) continue;
+      if (s_v[p] != lo) mask &= ~(1u << e);
+      else s_v[p] = word(w, p);
+    }
+    __syncthreads();
+  }
+  // rank the candidates among themselves by their remaining words
+#pragma unroll 4
+  for (int e = 0; e < WG_E; e++) {
+    if (!((mask >> e) & 1u)) continue;
+    const uint32_t x = s_v[e * WG_NT + tid];
+    if (x < lo || x > hi) continue;
+    const uint32_t i = atomicAdd(&s_ncand, 1u);
+    s_cval[i] = x;
+    s_cpos[i] = (uint32_t)(e * WG_NT + tid);
+  }
+  __syncthreads();
+  if ((uint32_t)tid < cnt) {
+    const uint32_t mine = s_cval[tid];
+    const int p = (int)s_cpos[tid];
+    uint32_t r = 0;
+    for (uint32_t j = 0; j < cnt; j++) {
+      const uint32_t o = s_cval[j];
+      bool less = o < mine;
+      if (o == mine && (int)j != tid) {
+        const int q = (int)s_cpos[j];
+        for (int x = w + 1; x <= clen; x++) {
+          const uint32_t a = word(x, q), b = word(x, p);
+          if (a != b) {
+            less = a < b;
+            break;
+          }
+        }
+      }
+      r += less ? 1u : 0u;
+    }
+    if (r == rem) s_pivot = p;
+  }
+  __syncthreads();
+  const int piv = s_pivot;
+  if (tid <= clen) s_pw[tid] = tid == 0 ? key[piv] : word(tid, piv);
+  __syncthreads();
+  const uint32_t pk = s_pw[0];
+  if (EXPLICIT && tid == 0) {
+    s_st.fixed[0] = pk;
+    write_child_domains(s_st, st + tr.cseg, s, L, isf);
+    s_cdim[0] = st[tr.cseg + 2 * s].dim;
+    s_cdim[1] = st[tr.cseg + 2 * s + 1].dim;
+  } else if (!EXPLICIT && tid < 2) {
+    s_cdim[tid] = (uint32_t)((level + 1) % D);
+  }
+  // sides, and ranks in (item, wave, lane) order
+  uint32_t lefts = 0, rights = 0;
+#pragma unroll 2
+  for (int e = 0; e < WG_E; e++) {
+    if (e * WG_NT >= m) {
+      if (lane == 0) s_cnt[e * NW + wave] = s_cnt[WG_E * NW + e * NW + wave] = 0u;
+      continue;
+    }
+    const int p = e * WG_NT + tid;
+    bool l = false, r = false;
+    if (p < m && p != piv) {
+      const uint32_t ke = w == 0 ? s_v[p] : key[p];
+      l = ke < pk;
+      if (ke == pk)
+        for (int x = 1; x <= clen; x++) {
+          const uint32_t a = word(x, p);
+          if (a != s_pw[x]) {
+            l = a < s_pw[x];
+            break;
+          }
+        }
+      r = !l;
+    }
+    const uint64_t ml = __ballot(l), mr = __ballot(r);
+    const uint64_t mine = l ? ml : mr;
+    s_rank[p] = (uint8_t)__builtin_amdgcn_mbcnt_hi((unsigned)(mine >> 32),
+                                                   __builtin_amdgcn_mbcnt_lo((unsigned)mine, 0u));
+    lefts |= l ? 1u << e : 0u;
+    rights |= r ? 1u << e : 0u;
+    if (lane == 0) {
+      s_cnt[e * NW + wave] = (uint32_t)__popcll(ml);
+      s_cnt[WG_E * NW + e * NW + wave] = (uint32_t)__popcll(mr);
+    }
+  }
+  __syncthreads();
+  {
+    static_assert(2 * WG_E * NW <= WG_NT, "a count per thread");
+    const uint32_t c = tid < 2 * WG_E * NW ? s_cnt[tid] : 0u;
+    const uint32_t pre = rk_block_scan<WG_NT>(c, s_wsum);
+    // the left counts come first: the right ones start behind all of them
+    if (tid < 2 * WG_E * NW)
+      s_cnt[tid] = tid < WG_E * NW ? pre : pre - (uint32_t)subtree_size(2 * node + 1, tr.n);
+  }
+  __syncthreads();
+  const int W = L.stride >> 2, cw0 = L.point_offset >> 2;
+  const int base0 = gn.offset(2 * s), base1 = gn.offset(2 * s + 1);
+  const uint32_t cd0 = s_cdim[0], cd1 = s_cdim[1];
+  // WG_BATCH elements at a time, all their loads in flight before a store
+  enum { WG_BATCH = 4 };
+  for (int e0 = 0; e0 < WG_E; e0 += WG_BATCH) {
+    if (e0 * WG_NT >= m) break;
+    uint32_t x[WG_BATCH][SW > 0 ? SW : 1], id[WG_BATCH];
+    int dst[WG_BATCH];
+    bool left[WG_BATCH];
+#pragma unroll
+    for (int i = 0; i < WG_BATCH; i++) {
+      const int e = e0 + i, p = e * WG_NT + tid;
+      left[i] = (lefts >> e) & 1u;
+      const bool mv = left[i] || ((rights >> e) & 1u);
+      dst[i] = -1;
+      id[i] = 0;
+      if (mv) {
+        id[i] = idx[p];
+        dst[i] = (left[i] ? base0 : base1) +
+                 (int)s_cnt[(left[i] ? 0 : WG_E * NW) + e * NW + wave] + s_rank[e * WG_NT + tid];
+      }
+#pragma unroll
+      for (int j = 0; j < SW; j++)
+        x[i][j] = mv && j < W ? ((const uint32_t *)(data + (size_t)p * L.stride))[j] : 0u;
+    }
+#pragma unroll
+    for (int i = 0; i < WG_BATCH; i++) {
+      if (dst[i] < 0) continue;
+      uint32_t *to = (uint32_t *)(ndata + (size_t)dst[i] * L.stride);
+      const int kw = cw0 + (int)(left[i] ? cd0 : cd1);
+      uint32_t kv = 0;
+      if (SW > 0) {
+#pragma unroll
+        for (int j = 0; j < SW; j++) {
+          if (j < W) to[j] = x[i][j];
+          kv = j == kw ? x[i][j] : kv;
+        }
+      } else {
+        const uint32_t *src = (const uint32_t *)(data + (size_t)((e0 + i) * WG_NT + tid) * L.stride);
+        for (int j = 0; j < W; j++) to[j] = src[j];
+        kv = src[kw];
+      }
+      nidx[dst[i]] = id[i];
+      if (tr.more) nkey[dst[i]] = ordered_key(kv, isf);
+    }
+  }
+  if (tid < W)
+    ((uint32_t *)(out + ((size_t)tr.base + node) * L.stride))[tid] =
+        patch_dim_word(((const uint32_t *)(data + (size_t)piv * L.stride))[tid], tid, L, dim);
+}
+
+// ---------------------------------------------------------------------------
 // host orchestration
 // ---------------------------------------------------------------------------
 
@@ -2156,6 +2457,14 @@ int make_forest_plan(ForestPlan &P, const long long *off, int ntrees, const cukd
       hseg += 1 << l;
       v.push_back(x);
     }
+    // the largest subtree of every tree is its first
+    bool wg = true;
+    for (const LvlTree &x : v) {
+      LevelGeom g;
+      g.init(x.n, l);
+      wg = wg && g.size(0) <= WG_MAX;
+    }
+    P.lvl_wg.push_back(wg ? 1 : 0);
     P.lvl.push_back(v);
     P.lvl_segs.push_back(hseg);
     P.lvl_stiles.push_back(stl);
@@ -2322,11 +2631,14 @@ int forest_build_run(const ForestPlan &P, void *d_points, void *d_bounds, uint8_
                        (int)P.in.size(), (const uint32_t *)acc, (uint32_t *)d_bounds, st, L,
                        expl ? 1 : 0);
   }
-  hipLaunchKernelGGL(k_copy_in, dim3(P.in_tiles), dim3(256), 0, s, in, dataA, idxA,
+  // levels from 'wg0' on run one workgroup per subtree
+  int wg0 = P.max_L0;
+  while (wg0 > 0 && P.lvl_wg[wg0 - 1]) wg0--;
+  hipLaunchKernelGGL(k_copy_in, dim3(P.in_tiles), dim3(COPY_NT), 0, s, in, dataA, idxA,
                      P.max_L0 > 0 ? keyA : (uint32_t *)nullptr, (const uint8_t *)pts, L,
                      (const SegState *)st, expl ? 1 : 0, h0,
-                     P.max_L0 > 0 ? (P.zero_end - P.off_hist) / 4 : 0);
-  if (P.max_L0 > 0) {
+                     wg0 > 0 ? (P.zero_end - P.off_hist) / 4 : 0);
+  if (wg0 > 0) {
     const TreeSet<LvlTree> set0 = make_set(P, ws, P.tables ? P.off_tab_lvl[0] : 0, P.lvl[0]);
     hipLaunchKernelGGL(k_level_init, dim3((P.lvl_segs[0] + 255) / 256), dim3(256), 0, s, set0,
                        P.lvl_segs[0], st, curp[0], tbp[0], 0, D, expl ? 1 : 0);
@@ -2336,6 +2648,19 @@ int forest_build_run(const ForestPlan &P, void *d_points, void *d_bounds, uint8_
   for (int level = 0; level < P.max_L0; level++) {
     const TreeSet<LvlTree> set =
         make_set(P, ws, P.tables ? P.off_tab_lvl[level] : 0, P.lvl[level]);
+    if (level >= wg0) {
+      const int W = L.stride >> 2;
+      auto kw = expl ? (W <= 5 ? k_level_wg<true, 5> : k_level_wg<true, 0>)
+                     : (W <= 3 ? k_level_wg<false, 3>
+                               : (W <= 5 ? k_level_wg<false, 5> : k_level_wg<false, 0>));
+      hipLaunchKernelGGL(kw, dim3(P.lvl_segs[level]), dim3(WG_NT), 0, s, set, level,
+                         (const uint32_t *)kcur, (const uint8_t *)dcur, (const uint32_t *)icur, st,
+                         dnext, inext, knext, pts, L);
+      uint8_t *t8 = dcur; dcur = dnext; dnext = t8;
+      uint32_t *t32 = icur; icur = inext; inext = t32;
+      t32 = kcur; kcur = knext; knext = t32;
+      continue;
+    }
     const int par = level & 1;
     const int hcopies = P.lvl_hcopies[level];
     // key word 0 (the split coordinate) over the whole level, one digit

@@ -50,6 +50,7 @@ struct ForestPlan {
   int max_L0 = 0;
   std::vector<std::vector<LvlTree>> lvl;  // per top level: the trees still on it
   std::vector<int> lvl_segs, lvl_stiles, lvl_ptiles;
+  std::vector<int> lvl_wg;  // every subtree of the level fits one workgroup (k_level_wg)
   std::vector<int> lvl_hcopies;  // digit histogram copies per subtree, per top level
   std::vector<FinTree> fin[5];            // per finish capacity 512 .. 8192
   int fin_blocks[5] = {0, 0, 0, 0, 0};
