@@ -2761,14 +2761,21 @@ size_t build_temp_bytes(int n, const cukd_layout &L)
   return P.total;
 }
 
+// screen: begun by the caller; its result is awaited behind the plan and the
+// allocation, before anything is written
 int build_tree_impl(void *d_points, int n, const cukd_layout &L, void *d_bounds, hipStream_t s,
-                    const MemResource &mem)
+                    const MemResource &mem, NanScreen &screen)
 {
   ForestPlan P;
   const long long off[2] = {0, n};
   make_forest_plan(P, off, 1, L, false);
   uint8_t *ws = nullptr;
-  if (mem.alloc((void **)&ws, P.total, s) != 0) return CUKD_ERR_ALLOC;
+  const int ac = mem.alloc((void **)&ws, P.total, s);
+  if (int nc = screen.end()) {
+    if (ac == 0) mem.release(ws, s);
+    return nc;
+  }
+  if (ac != 0) return CUKD_ERR_ALLOC;
   const int rc = forest_build_run(P, d_points, d_bounds, ws, s);
   mem.release(ws, s);
   return rc;

@@ -118,11 +118,10 @@ int build_tree_tl(void *d_points, int n, const cukd_layout &L, void *d_bounds, h
                   const MemResource &mem, bool carry_rank);
 size_t build_tl_temp_bytes(int n, const cukd_layout &L, bool carry_rank);
 int build_tree_impl(void *d_points, int n, const cukd_layout &L, void *d_bounds,
-                    hipStream_t s, const MemResource &mem);
+                    hipStream_t s, const MemResource &mem, NanScreen &screen);
 size_t build_temp_bytes(int n, const cukd_layout &L);
 int build_bounds_only(void *d_bounds, const void *d_points, int n, const cukd_layout &L,
                       hipStream_t s);
-int screen_nan(const void *d_points, int n, const cukd_layout &L, hipStream_t stream);
 
 size_t query_order_temp_bytes(int nq);
 int32_t *make_query_order(void *tmp, const float *q, int nq, int D, hipStream_t s);
@@ -275,12 +274,15 @@ int cukd_build_tree(void *d_points, int32_t n, const cukd_layout *layout, int bu
                    "but no memory for world bounds provided");
     return CUKD_ERR_NO_BOUNDS;
   }
-  if (int rc = screen_nan(d_points, n, *layout, stream)) return rc;
+  NanScreen screen;
+  if (int rc = screen.begin(d_points, n, *layout, stream)) return rc;
   MemResource mr{mem};
-  if (builder == CUKD_BUILDER_ID_BITONIC || builder == CUKD_BUILDER_ID_INPLACE)
+  if (builder == CUKD_BUILDER_ID_BITONIC || builder == CUKD_BUILDER_ID_INPLACE) {
+    if (int rc = screen.end()) return rc;
     return build_tree_tl(d_points, n, *layout, d_world_bounds, stream, mr,
                          builder == CUKD_BUILDER_ID_BITONIC);
-  return build_tree_impl(d_points, n, *layout, d_world_bounds, stream, mr);
+  }
+  return build_tree_impl(d_points, n, *layout, d_world_bounds, stream, mr, screen);
 }
 
 int cukd_build_tree_host(void *h_points, int32_t n, const cukd_layout *layout,
@@ -739,7 +741,9 @@ int cukd_spatial_build(cukd_spatial_tree *tree, const void *d_points, int32_t n,
     set_last_error("leaf threshold %d exceeds the 16-bit leaf count", leaf_threshold);
     return CUKD_ERR_INVALID;
   }
-  if (int rc = screen_nan(d_points, n, *layout, stream)) return rc;
+  NanScreen screen;
+  if (int rc = screen.begin(d_points, n, *layout, stream)) return rc;
+  if (int rc = screen.end()) return rc;
   MemResource mr{mem};
   return spatial_build_impl(tree, d_points, n, *layout, leaf_threshold, stream, mr);
 }

@@ -172,6 +172,15 @@ void clear_last_error();
 int forest_num_dims(const cukd_forest *f);
 int forest_num_trees(const cukd_forest *f);
 
+// NaN screen of a single-tree build (nan_screen.hip).  Every begin() that
+// returns CUKD_OK is followed by end() before the points are written.
+struct NanScreen {
+  int slot = -1;
+  hipStream_t stream = nullptr;
+  int begin(const void *d_points, int n, const cukd_layout &L, hipStream_t s);
+  int end();
+};
+
 struct MemResource {
   const cukd_mem_resource *user;
   int alloc(void **p, size_t bytes, hipStream_t s) const;

@@ -5,13 +5,13 @@
 // (builder_thrust.h:401-404), which is no strict weak order once a NaN is
 // present, so its result is undefined there.  cukd_build_tree screens the
 // coordinates first and returns CUKD_ERR_INVALID, leaving the array as it
-// was.  The result word of each call lives in a library-owned device array
-// (one 256-byte line per slot), so no builder, the in-place one included,
-// allocates for it.  A free slot's word is zero: it starts so, a scan only
-// sets it, and a call that found a NaN writes zero back before it frees
-// the slot.
+// was.  The result word of each call lives in pinned host memory of the
+// library's own (one 256-byte line per slot, allocated once), so no builder,
+// the in-place one included, allocates device memory for it, and reading it
+// needs no copy: the scan stores to it only where it finds a NaN, and the
+// wait for the stream makes that store visible.  The scan and the wait are
+// two calls, so that a builder plans and allocates while the scan runs.
 #include <condition_variable>
-#include <map>
 #include <mutex>
 
 #include "cukd_common.h"
@@ -19,8 +19,6 @@
 namespace cukd_amd {
 
 enum { NAN_SLOTS = 64, NAN_SLOT_WORDS = 64 };
-
-static __device__ __align__(256) uint32_t g_nan_slots[NAN_SLOTS * NAN_SLOT_WORDS];
 
 
 // One thread per element (grid-stride): any NaN coordinate sets the flag.
@@ -43,22 +41,23 @@ namespace {
 
 std::mutex g_mu;
 std::condition_variable g_cv;
-uint64_t g_busy = 0;                  // slots in use, one bit each
-std::map<int, uint32_t *> g_base;     // device -> address of g_nan_slots
+uint64_t g_busy = 0;       // slots in use, one bit each
+uint32_t *g_slots = nullptr;  // pinned host memory, readable by every device
 
-// device address of this device's copy of the slot array
 int slot_base(uint32_t **base)
 {
-  int dev = 0;
-  CUKD_HIP(hipGetDevice(&dev));
   std::lock_guard<std::mutex> lk(g_mu);
-  auto it = g_base.find(dev);
-  if (it == g_base.end()) {
+  if (!g_slots) {
+#ifdef hipHostMallocPortable
+    const unsigned flags = hipHostMallocPortable | hipHostMallocMapped | hipHostMallocCoherent;
+#else
+    const unsigned flags = hipHostMallocDefault;
+#endif
     void *p = nullptr;
-    CUKD_HIP(hipGetSymbolAddress(&p, HIP_SYMBOL(g_nan_slots)));
-    it = g_base.emplace(dev, (uint32_t *)p).first;
+    CUKD_HIP(hipHostMalloc(&p, NAN_SLOTS * NAN_SLOT_WORDS * 4, flags));
+    g_slots = (uint32_t *)p;
   }
-  *base = it->second;
+  *base = g_slots;
   return CUKD_OK;
 }
 
@@ -82,32 +81,40 @@ void give_slot(int s)
 
 }  // namespace
 
-// CUKD_OK when no coordinate is NaN (and for int layouts), CUKD_ERR_INVALID
-// when one is.  Synchronises 'stream'.  Under stream capture the screen is
-// skipped (a capture cannot wait for a result), and CUKD_OK is returned.
-int screen_nan(const void *d_points, int n, const cukd_layout &L, hipStream_t stream)
+// Launches the scan.  Under stream capture nothing is screened (a capture
+// cannot wait for a result), nor for int layouts.
+int NanScreen::begin(const void *d_points, int n, const cukd_layout &L, hipStream_t s)
 {
   if (L.scalar_type != CUKD_SCALAR_F32 || n < 1) return CUKD_OK;
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-  CUKD_HIP(hipStreamIsCapturing(stream, &cs));
+  CUKD_HIP(hipStreamIsCapturing(s, &cs));
   if (cs != hipStreamCaptureStatusNone) return CUKD_OK;
   uint32_t *base = nullptr;
   if (int rc = slot_base(&base)) return rc;
-  const int slot = take_slot();
-  uint32_t *flag = base + slot * NAN_SLOT_WORDS;
-  uint32_t h = 0;
+  stream = s;
+  slot = take_slot();
+  volatile uint32_t *flag = base + slot * NAN_SLOT_WORDS;
+  *flag = 0u;
   const long long blocks = ((long long)n + 255) / 256;
-  hipLaunchKernelGGL(k_nan_scan, dim3((unsigned)(blocks < 4096 ? blocks : 4096)), dim3(256), 0,
-                     stream, (const uint8_t *)d_points, (long long)n, L, flag);
-  hipError_t e = hipGetLastError();
-  if (e == hipSuccess) e = hipMemcpyAsync(&h, flag, 4, hipMemcpyDeviceToHost, stream);
-  if (e == hipSuccess) e = hipStreamSynchronize(stream);
-  if (e == hipSuccess && h) {
-    const uint32_t zero = 0u;
-    e = hipMemcpyAsync(flag, &zero, 4, hipMemcpyHostToDevice, stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(stream);
-  }
+  hipLaunchKernelGGL(k_nan_scan, dim3((unsigned)(blocks < 4096 ? blocks : 4096)), dim3(256), 0, s,
+                     (const uint8_t *)d_points, (long long)n, L, base + slot * NAN_SLOT_WORDS);
+  const hipError_t e = hipGetLastError();
+  if (e == hipSuccess) return CUKD_OK;
   give_slot(slot);
+  slot = -1;
+  set_last_error("NaN screen failed: %s", hipGetErrorString(e));
+  return CUKD_ERR_HIP;
+}
+
+// Waits for the scan: CUKD_OK when no coordinate is NaN, CUKD_ERR_INVALID when
+// one is.
+int NanScreen::end()
+{
+  if (slot < 0) return CUKD_OK;
+  const hipError_t e = hipStreamSynchronize(stream);
+  const uint32_t h = *(volatile uint32_t *)(g_slots + slot * NAN_SLOT_WORDS);
+  give_slot(slot);
+  slot = -1;
   if (e != hipSuccess) {
     set_last_error("NaN screen failed: %s", hipGetErrorString(e));
     return CUKD_ERR_HIP;
