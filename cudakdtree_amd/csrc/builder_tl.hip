@@ -13,7 +13,7 @@
 // is a stable sort -- the host builder's chain, ties included.  The sort is
 // an all-ascending bitonic network (mirror step, then half-cleaners; +inf
 // padding never moves) run as global compare-exchange passes for large
-// strides and LDS tile passes for small ones; once subtrees fit in LDS, one
+// strides (up to three steps each) and LDS tile passes for small ones; once subtrees fit in LDS, one
 // workgroup per subtree finishes all remaining levels.
 //
 //  * bitonic: the rank travels with each element in an N-int array, so the
@@ -189,6 +189,129 @@ __global__ void k_tl_cx(int level, int n, int half_p, int ks, int j, int mirror,
   if (tl_greater<CARRY>(ea, ua, eb, ub, dim, L, isf)) {
     swap_elems(ea, eb, L.stride >> 2);
     if (CARRY) { rank[plo] = ub; rank[phi] = ua; }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// up to three consecutive global steps in one pass: a thread holds the 2^R
+// elements that R strides connect, in registers
+// ---------------------------------------------------------------------------
+// mirror: the mirror step of block size ks, then R - 1 half-cleaners (strides
+// ks/4, ks/8): the lower half's elements o + a q (q = ks / 2^R) and their
+// mirror images.  Otherwise the half-cleaners of strides j, j/2, j/4.  The
+// steps and their order are those of the one-step passes, so the sorted order
+// is the same.  Each pass is bound by its trip through memory and its launch,
+// about 7.5 us for 1M float3 however many steps it makes: 216 one-step passes
+// took 1612 us of the in-place build's 3575; with up to three steps each the
+// build takes 2849 us.  Four would need 16 elements in registers, 48 words and
+// more.  SW: elements of at most SW words.
+template <bool CARRY, bool EXPLICIT, int SW, int R>
+__global__ __launch_bounds__(256) void k_tl_cxr(int level, int n, int half_p, int ks, int j,
+                                                int mirror, uint8_t *data, uint32_t *rank,
+                                                cukd_layout L)
+{
+  enum { N = 1 << R, H = N / 2 };
+  const int groups = half_p / H;  // per subtree
+  const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  const int gl = (int)(t / groups);
+  const int i = (int)(t - (long long)gl * groups);
+  if (gl >= (1 << level)) return;
+  const int g = (1 << level) - 1 + gl;
+  const int size = subtree_size(g, n), left = subtree_size(2 * g + 1, n);
+  int v[N];
+  if (mirror) {
+    const int q = ks >> R, b = i / q, o = i - b * q;
+#pragma unroll
+    for (int a = 0; a < H; a++) {
+      v[a] = b * ks + o + a * q;
+      v[H + a] = b * ks + ks - 1 - o - a * q;
+    }
+  } else {
+    const int q = j >> (R - 1), hi = i / q;
+#pragma unroll
+    for (int a = 0; a < N; a++) v[a] = hi * 2 * j + (i - hi * q) + a * q;
+  }
+  const int W = L.stride >> 2, cw0 = L.point_offset >> 2;
+  const bool isf = L.scalar_type == CUKD_SCALAR_F32;
+  int dim = level % L.num_dims;
+  uint32_t x[N][SW], key[N], u[N];
+  int pos[N];
+#pragma unroll
+  for (int a = 0; a < N; a++) {
+    pos[a] = v[a] < size ? v_pos(g, v[a], left) : -1;
+    u[a] = CARRY && pos[a] >= 0 ? rank[pos[a]] : 0u;
+    const uint32_t *e = (const uint32_t *)(data + (size_t)(pos[a] < 0 ? 0 : pos[a]) * L.stride);
+#pragma unroll
+    for (int w = 0; w < SW; w++) x[a][w] = pos[a] >= 0 && w < W ? e[w] : 0u;
+  }
+  if (pos[0] < 0) return;  // the smallest index: the others are past the end too
+  if (EXPLICIT) dim = read_dim_field(data + (size_t)pos[0] * L.stride, L);
+#pragma unroll
+  for (int a = 0; a < N; a++) {
+    uint32_t c = 0;
+#pragma unroll
+    for (int w = 0; w < SW; w++) c = w == cw0 + dim ? x[a][w] : c;
+    key[a] = ordered_key(c, isf);
+  }
+  bool moved = false;
+  // slot a holds the lower index of the two
+  auto step = [&](int a, int b) {
+    if (pos[a] < 0 || pos[b] < 0) return;
+    bool gt = key[a] > key[b];
+    if (key[a] == key[b]) {
+      if (CARRY) {
+        gt = u[a] > u[b];
+      } else {
+        bool same = true;
+#pragma unroll
+        for (int w = 0; w < SW; w++) {
+          gt = same && w < W ? x[a][w] > x[b][w] : gt;
+          same = same && (w >= W || x[a][w] == x[b][w]);
+        }
+      }
+    }
+    if (!gt) return;
+    moved = true;
+#pragma unroll
+    for (int w = 0; w < SW; w++) {
+      const uint32_t y = x[a][w];
+      x[a][w] = x[b][w];
+      x[b][w] = y;
+    }
+    uint32_t y = key[a];
+    key[a] = key[b];
+    key[b] = y;
+    y = u[a];
+    u[a] = u[b];
+    u[b] = y;
+  };
+  if (mirror) {
+#pragma unroll
+    for (int a = 0; a < H; a++) step(a, H + a);
+#pragma unroll
+    for (int bit = H / 2; bit > 0; bit >>= 1)
+#pragma unroll
+      for (int a = 0; a < H; a++)
+        if (!(a & bit)) {
+          step(a, a | bit);
+          step(H + (a | bit), H + a);  // the upper half runs downwards
+        }
+  } else {
+#pragma unroll
+    for (int bit = H; bit > 0; bit >>= 1)
+#pragma unroll
+      for (int a = 0; a < N; a++)
+        if (!(a & bit)) step(a, a | bit);
+  }
+  if (!moved) return;
+#pragma unroll
+  for (int a = 0; a < N; a++) {
+    if (pos[a] < 0) continue;
+    uint32_t *e = (uint32_t *)(data + (size_t)pos[a] * L.stride);
+#pragma unroll
+    for (int w = 0; w < SW; w++)
+      if (w < W) e[w] = x[a][w];
+    if (CARRY) rank[pos[a]] = u[a];
   }
 }
 
@@ -411,11 +534,56 @@ static hipError_t launch_tl_finish(bool expl, int blocks, size_t dyn, hipStream_
 // top levels: per level, sort every subtree's T-element tiles in LDS, then
 // merge them with global compare-exchange passes (strides >= T) and LDS tile
 // passes (strides < T)
+// One to three steps in one launch (k_tl_cxr), for elements of up to 5 words.
+template <bool CARRY, bool EXPLICIT, int SW>
+static void launch_cxr(int steps, long long pairs, int level, int n, int half_p, int ks, int j,
+                       int mirror, uint8_t *data, uint32_t *rank, const cukd_layout &L,
+                       hipStream_t s)
+{
+  const long long threads = pairs >> (steps - 1);
+  const dim3 blocks((unsigned)((threads + 255) / 256));
+  if (steps == 3)
+    hipLaunchKernelGGL((k_tl_cxr<CARRY, EXPLICIT, SW, 3>), blocks, dim3(256), 0, s, level, n,
+                       half_p, ks, j, mirror, data, rank, L);
+  else if (steps == 2)
+    hipLaunchKernelGGL((k_tl_cxr<CARRY, EXPLICIT, SW, 2>), blocks, dim3(256), 0, s, level, n,
+                       half_p, ks, j, mirror, data, rank, L);
+  else
+    hipLaunchKernelGGL((k_tl_cxr<CARRY, EXPLICIT, SW, 1>), blocks, dim3(256), 0, s, level, n,
+                       half_p, ks, j, mirror, data, rank, L);
+}
+
+// the steps of merge ks with strides of at least T
+template <bool CARRY, bool EXPLICIT>
+static void launch_steps(long long pairs, int level, int n, int half_p, int ks, int T,
+                         uint8_t *data, uint32_t *rank, const cukd_layout &L, hipStream_t s)
+{
+  const int W = L.stride >> 2;
+  int left = 1;  // the mirror step and the half-cleaners ks/4 .. T
+  for (int j = ks >> 2; j >= T; j >>= 1) left++;
+  int mirror = 1, j = 0;
+  while (left > 0) {
+    // wide elements take one step a launch
+    const int steps = W > 5 ? 1 : left < 3 ? left : 3;
+    if (W > 5) {
+      hipLaunchKernelGGL((k_tl_cx<CARRY, EXPLICIT>), dim3((unsigned)((pairs + 255) / 256)),
+                         dim3(256), 0, s, level, n, half_p, ks, j, mirror, data, rank, L);
+    } else if (W <= 3) {
+      launch_cxr<CARRY, EXPLICIT, 3>(steps, pairs, level, n, half_p, ks, j, mirror, data, rank, L, s);
+    } else {
+      launch_cxr<CARRY, EXPLICIT, 5>(steps, pairs, level, n, half_p, ks, j, mirror, data, rank, L, s);
+    }
+    left -= steps;
+    j = mirror ? ks >> (steps + 1) : j >> steps;
+    mirror = 0;
+  }
+}
+
 template <bool CARRY, bool EXPLICIT, int T>
 static hipError_t tl_levels(int n, int L0, uint8_t *data, uint32_t *rank, const uint32_t *world,
                             const cukd_layout &L, hipStream_t s)
 {
-  enum { NT = 256 };
+  enum { NT = T >= 2048 ? 512 : 256 };
   const size_t dyn = (size_t)T * L.stride;
   hipError_t e = hipFuncSetAttribute((const void *)k_tl_tile<CARRY, EXPLICIT, T, NT>,
                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)dyn);
@@ -435,15 +603,10 @@ static hipError_t tl_levels(int n, int L0, uint8_t *data, uint32_t *rank, const 
     hipLaunchKernelGGL((k_tl_tile<CARRY, EXPLICIT, T, NT>), dim3(segs * tiles), dim3(NT), dyn, s,
                        level, n, tiles, 0, 1, data, rank, L);
     const long long pairs = (long long)segs * (P / 2);
-    const unsigned blocks = (unsigned)((pairs + 255) / 256);
-    for (int ks = 2 * T; ks <= P; ks <<= 1) {
-      hipLaunchKernelGGL((k_tl_cx<CARRY, EXPLICIT>), dim3(blocks), dim3(256), 0, s, level, n,
-                         P / 2, ks, 0, 1, data, rank, L);
-      for (int j = ks >> 2; j >= T; j >>= 1)
-        hipLaunchKernelGGL((k_tl_cx<CARRY, EXPLICIT>), dim3(blocks), dim3(256), 0, s, level, n,
-                           P / 2, ks, j, 0, data, rank, L);
+    for (long long ks = 2 * T; ks <= P; ks <<= 1) {
+      launch_steps<CARRY, EXPLICIT>(pairs, level, n, P / 2, (int)ks, T, data, rank, L, s);
       hipLaunchKernelGGL((k_tl_tile<CARRY, EXPLICIT, T, NT>), dim3(segs * tiles), dim3(NT), dyn,
-                         s, level, n, tiles, ks, 0, data, rank, L);
+                         s, level, n, tiles, (int)ks, 0, data, rank, L);
     }
   }
   return hipGetLastError();
@@ -453,7 +616,10 @@ template <bool CARRY, bool EXPLICIT>
 static hipError_t tl_levels_for_stride(int n, int L0, uint8_t *data, uint32_t *rank,
                                        const uint32_t *world, const cukd_layout &L, hipStream_t s)
 {
-  // tiles of at most 48 KiB of elements
+  // tiles of at most 48 KiB of elements.  2048 up to 20 bytes: a step less per
+  // merge through memory (1M float3 in place: 2541 us; 1024: 2849, 4096, which
+  // leaves two workgroups per CU: 2961)
+  if (L.stride <= 20) return tl_levels<CARRY, EXPLICIT, 2048>(n, L0, data, rank, world, L, s);
   if (L.stride <= 48) return tl_levels<CARRY, EXPLICIT, 1024>(n, L0, data, rank, world, L, s);
   if (L.stride <= 96) return tl_levels<CARRY, EXPLICIT, 512>(n, L0, data, rank, world, L, s);
   return tl_levels<CARRY, EXPLICIT, 256>(n, L0, data, rank, world, L, s);
