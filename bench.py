@@ -943,8 +943,8 @@ def main():
     e1.record(stream)
     torch.cuda.synchronize()
     kernel_ms = e0.elapsed_time(e1) / args.steps
-    # the same launch with one query per lane (the kernel the default
-    # two-per-lane one replaces), for comparison
+    # the same launch with the kernel that does not prune by box, for
+    # comparison
     for _ in range(args.warmup):
         ck.knn(tree, lay, qs, k, out=out, flags=ck.QUERY_ONE_PER_LANE | ck.QUERY_PRESORTED)
     torch.cuda.synchronize()
@@ -1087,9 +1087,9 @@ def main():
                      "unit": "GB/s", "frac": round(knn_gbs / HBM_PEAK_GBS, 4),
                      "traffic": traffic,
                      "traffic_source": traffic_note,
-                     "kernel": "k_query2s<3, FixedCandidateList<8>> (stack-based, two queries "
-                               "per lane, pending plane distances in LDS) on Morton-ordered "
-                               "queries",
+                     "kernel": "k_query_box<3, stack-based, RegSorted<8>> (box-pruned, "
+                               "pending plane distances in LDS, list in registers) on "
+                               "Morton-ordered queries; bytes of the unpruned visits",
                      "algorithmic_bytes_per_launch": knn_bytes,
                      "avg_launch_ms": round(kernel_ms, 4),
                      "step_ms_with_ordering": round(ev_ms, 4)},

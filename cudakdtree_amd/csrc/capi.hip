@@ -372,7 +372,7 @@ int log2_bucket(int n)
 // Launches the query in a (order unset).  CUKD_QUERY_SORT: Morton-ordered
 // launch.  CUKD_QUERY_AUTOTUNE: the first call per (dims, traversal, list,
 // k, log2 nq, forest) times workgroup sizes 64/128/256 with and without
-// ordering, and one or two queries per lane where the kernel allows two,
+// ordering, and with and without box pruning where the kernel allows it,
 // on these very inputs (every variant writes identical results),
 // synchronising the stream once, and caches the fastest; later calls use
 // the cache.  repeatable = false (multi-round lists) only reads the cache.
