@@ -6,7 +6,7 @@
 // nodes at once.  Both give the same tree:
 //   decide   : leaf if count <= threshold, else split the widest centroid
 //              extent at its centre (ties pick the earlier dim; a centre
-//              equal to either end makes a degenerate "dim -1" split)
+//              not between the ends makes a degenerate "dim -1" split)
 //   number   : children of this round's split nodes get consecutive ids in
 //              ascending parent order (exclusive scan; the reference takes
 //              atomicAdd order, so its numbering is not reproducible)
@@ -206,7 +206,36 @@ __global__ __launch_bounds__(256) void k_sp_root_bounds(SpNode *nodes, const uin
   }
 }
 
-// selectSplits (spatial-kdtree.h:316-396) for the open nodes [a, b)
+// selectSplits' rule (spatial-kdtree.h:316-396): the widest extent at its
+// centre, ties to the earlier dim; -1 (the points are dealt out in turn) where
+// the centre is not strictly between the extent's ends.  The reference looks
+// for a centre equal to an end only, and its build never ends where the sum of
+// the ends overflows or is NaN: one child would keep every point.  The halves
+// are added instead where the sum overflows, so both children of any split
+// have points, which bounds the nodes of a subtree of m points by 2 m - 1.
+// box(w): lower ends, then upper ends, encoded.
+template <class F>
+__device__ inline int sp_choose(int D, F box, float &pos)
+{
+  float widest_w = 0.f;
+  int widest = -1;
+  for (int d = 0; d < D; d++) {
+    const float w = abox_dec(box(D + d)) - abox_dec(box(d));
+    if (w <= widest_w) continue;
+    widest_w = w;
+    widest = d;
+  }
+  if (widest >= 0) {
+    const float lo = abox_dec(box(widest)), hi = abox_dec(box(D + widest));
+    pos = 0.5f * (lo + hi);
+    if (isinf(pos)) pos = 0.5f * lo + 0.5f * hi;
+    if (!(pos > lo && pos < hi)) widest = -1;
+  }
+  if (widest < 0) pos = abox_dec(box(0));
+  return widest;
+}
+
+// selectSplits for the open nodes [a, b)
 __global__ void k_sp_decide(SpNode *nodes, uint32_t *split_flag, uint32_t *degen, int a, int b,
                             int D, uint32_t threshold)
 {
@@ -220,25 +249,10 @@ __global__ void k_sp_decide(SpNode *nodes, uint32_t *split_flag, uint32_t *degen
     t.dim = 0;
     t.pos = 0.f;
   } else {
-    float widest_w = 0.f;
-    int widest = -1;
-    for (int d = 0; d < D; d++) {
-      const float w = abox_dec(t.hi[d]) - abox_dec(t.lo[d]);
-      if (w <= widest_w) continue;
-      widest_w = w;
-      widest = d;
-    }
-    float pos = 0.f;
-    if (widest >= 0) {
-      const float lo = abox_dec(t.lo[widest]), hi = abox_dec(t.hi[widest]);
-      pos = 0.5f * (lo + hi);
-      if (pos == lo || pos == hi) widest = -1;
-    }
-    if (widest < 0) {
-      pos = abox_dec(t.lo[0]);
-      *degen = 1u;  // same value from every writer
-    }
-    t.dim = widest;
+    float pos;
+    const int dim = sp_choose(D, [&](int w) { return w < D ? t.lo[w] : t.hi[w - D]; }, pos);
+    if (dim < 0) *degen = 1u;  // same value from every writer
+    t.dim = dim;
     t.pos = pos;
     t.state = SP_SPLIT;
     is_split = 1;

@@ -60,28 +60,6 @@ struct SpLevelBase {
   uint32_t v[SPB_LEVELS + 1];
 };
 
-// selectSplits' rule (spatial-kdtree.h:316-396): the widest extent at its
-// centre, ties to the earlier dim; -1 where the centre meets an end
-template <class F>
-__device__ inline int sp_choose(int D, F box, float &pos)
-{
-  float widest_w = 0.f;
-  int widest = -1;
-  for (int d = 0; d < D; d++) {
-    const float w = abox_dec(box(D + d)) - abox_dec(box(d));
-    if (w <= widest_w) continue;
-    widest_w = w;
-    widest = d;
-  }
-  if (widest >= 0) {
-    const float lo = abox_dec(box(widest)), hi = abox_dec(box(D + widest));
-    pos = 0.5f * (lo + hi);
-    if (pos == lo || pos == hi) widest = -1;
-  }
-  if (widest < 0) pos = abox_dec(box(0));
-  return widest;
-}
-
 // exclusive scan over the NT threads of a workgroup; s_w: NT / 64 + 1 words.
 // The caller separates two uses of s_w by a barrier.
 template <int NT>

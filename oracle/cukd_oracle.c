@@ -818,9 +818,15 @@ int64_t oc_spatial_build(const void *points, int64_t n, const oc_layout *L,
       }
       float pos = 0.f;
       if (widest >= 0) {
-        pos = 0.5f * (abox_dec(t->lo[widest]) + abox_dec(t->hi[widest]));
-        if (pos == abox_dec(t->lo[widest]) || pos == abox_dec(t->hi[widest]))
-          widest = -1;
+        /* The centre of [lo, hi] splits only where it lies strictly between
+         * them.  The reference tests for an end alone; where lo + hi
+         * overflows, or is NaN, its split leaves one child as it was, and
+         * the build never ends.  Here the halves are added instead, and a
+         * centre that still is no number between the ends is degenerate. */
+        const float lo = abox_dec(t->lo[widest]), hi = abox_dec(t->hi[widest]);
+        pos = 0.5f * (lo + hi);
+        if (isinf(pos)) pos = 0.5f * lo + 0.5f * hi;
+        if (!(pos > lo && pos < hi)) widest = -1;
       }
       if (widest < 0) pos = abox_dec(t->lo[0]);
       t->dim = widest;

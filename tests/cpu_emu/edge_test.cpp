@@ -1,0 +1,151 @@
+// CPU kernel-emulator tests of edge cases of the C ABI (test infrastructure;
+// see emu_test.cpp): inputs, launches and runtime states that a GPU test
+// cannot or must not bring about.
+//
+//   edge_test [case-name-substring]
+#include <cmath>
+#include <cstdio>
+#include <cstring>
+#include <functional>
+#include <string>
+#include <vector>
+
+#include <hip/hip_runtime_api.h>
+
+#include "cukd_amd.h"
+#include "../../oracle/cukd_oracle.h"
+
+// query kernels are compiled for dims 2, 3 and 4 only
+namespace cukd_amd {
+struct QueryArgs;
+#define CUKD_EMU_NO_DIM(d)                                                          \
+  hipError_t launch_query_##d(int, const QueryArgs &, hipStream_t) { return hipErrorInvalidValue; }
+CUKD_EMU_NO_DIM(1)
+CUKD_EMU_NO_DIM(5)
+CUKD_EMU_NO_DIM(6)
+CUKD_EMU_NO_DIM(7)
+CUKD_EMU_NO_DIM(8)
+}  // namespace cukd_amd
+
+namespace {
+
+uint64_t sm(uint64_t &x)
+{
+  uint64_t z = (x += 0x9E3779B97F4A7C15ull);
+  z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
+  z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
+  return z ^ (z >> 31);
+}
+float unit(uint64_t &x) { return (float)(sm(x) >> 40) * (1.f / 16777216.f); }
+
+// device memory of a vector's size and contents
+template <class T> struct Dev {
+  T *p = nullptr;
+  size_t n;
+  explicit Dev(size_t n_) : n(n_) { hipMalloc((void **)&p, n * sizeof(T) + 4); }
+  explicit Dev(const std::vector<T> &v) : Dev(v.size()) { if (n) memcpy(p, v.data(), n * sizeof(T)); }
+  ~Dev() { hipFree(p); }
+  bool same(const std::vector<T> &v) const { return !n || !memcmp(p, v.data(), n * sizeof(T)); }
+};
+
+oc_layout ocl(const cukd_layout &L)
+{
+  return oc_layout{L.num_dims, L.scalar_type, L.stride, L.point_offset, L.dim_offset, L.dim_bytes};
+}
+cukd_layout floats(int D) { return cukd_layout{D, CUKD_SCALAR_F32, 4 * D, 0, -1, 4}; }
+
+struct SpatialRef {
+  std::vector<oc_spatial_node> nodes;
+  std::vector<uint32_t> prims;
+  std::vector<float> box;
+  SpatialRef(const std::vector<float> &pts, const cukd_layout &L, int leaf)
+  {
+    const int n = (int)pts.size() / L.num_dims;
+    const oc_layout O = ocl(L);
+    nodes.resize(oc_spatial_build(pts.data(), n, &O, leaf, nullptr, nullptr, nullptr));
+    prims.resize(n);
+    box.resize(2 * L.num_dims);
+    oc_spatial_build(pts.data(), n, &O, leaf, nodes.data(), prims.data(), box.data());
+  }
+  bool same(const cukd_spatial_tree &t) const
+  {
+    return (size_t)t.num_nodes == nodes.size() &&
+           !memcmp(t.nodes, nodes.data(), nodes.size() * sizeof(nodes[0])) &&
+           !memcmp(t.prim_ids, prims.data(), prims.size() * 4) &&
+           !memcmp(t.bounds, box.data(), box.size() * 4);
+  }
+};
+
+// Extents whose centre does not lie strictly between their ends as a float:
+// ends whose sum overflows, and infinite ones.
+bool spatial_centre_case(const char *kind, int n, int D, int leaf)
+{
+  uint64_t seed = 7 + n;
+  std::vector<float> pts((size_t)n * D);
+  for (int i = 0; i < n; i++)
+    for (int d = 0; d < D; d++) {
+      float v = unit(seed);
+      const uint32_t r = (uint32_t)(sm(seed) % 5);
+      if (!strcmp(kind, "sum overflows")) v = d == 0 ? 1.8e38f + 1.6e38f * v : v;
+      if (!strcmp(kind, "negative sum overflows")) v = -1.8e38f - 1.6e38f * v;
+      if (!strcmp(kind, "opposite infinities")) v = r == 0 ? -INFINITY : r == 1 ? INFINITY : v;
+      if (!strcmp(kind, "infinity in one dim")) v = d == D - 1 && r < 3 ? INFINITY : v;
+      if (!strcmp(kind, "minus infinity")) v = r < 2 ? -INFINITY : v;
+      if (!strcmp(kind, "all infinite")) v = r < 2 ? -INFINITY : INFINITY;
+      pts[(size_t)i * D + d] = v;
+    }
+  const cukd_layout L = floats(D);
+  const oc_layout O = ocl(L);
+  const SpatialRef ref(pts, L, leaf);
+  Dev<float> dp(pts);
+  cukd_spatial_tree t;
+  if (cukd_spatial_build(&t, dp.p, n, &L, leaf, nullptr, nullptr) != CUKD_OK) return false;
+  bool ok = ref.same(t);
+  // queries beside the points, at infinity and in the ordinary range
+  std::vector<float> q(pts.begin(), pts.begin() + (size_t)(n < 60 ? n : 60) * D);
+  for (int i = 0; i < 20 * D; i++) q.push_back(unit(seed));
+  const int nq = (int)q.size() / D, k = 5;
+  Dev<float> dq(q), dd((size_t)nq * k);
+  Dev<int32_t> di((size_t)nq * k);
+  std::vector<int32_t> ri((size_t)nq * k);
+  std::vector<float> rd((size_t)nq * k);
+  for (int m : {CUKD_STACK_BASED, CUKD_CCT}) {
+    oc_spatial_knn(m, OC_LIST_FIXED, k, ref.nodes.data(), ref.prims.data(), ref.box.data(),
+                   pts.data(), &O, q.data(), nq, INFINITY, ri.data(), rd.data(), nullptr, 1);
+    ok = ok && cukd_spatial_knn(m, CUKD_LIST_FIXED, k, &t, &L, dq.p, nq, INFINITY, di.p, dd.p,
+                                nullptr, nullptr) == CUKD_OK &&
+         di.same(ri) && dd.same(rd);
+  }
+  cukd_spatial_free(&t, nullptr, nullptr);
+  return ok;
+}
+
+}  // namespace
+
+int main(int argc, char **argv)
+{
+  const std::string only = argc > 1 ? argv[1] : "";
+  struct Case {
+    std::string name;
+    std::function<bool()> run;
+  };
+  std::vector<Case> cases;
+  for (const char *kind : {"sum overflows", "negative sum overflows", "opposite infinities",
+                           "infinity in one dim", "minus infinity", "all infinite"})
+    for (int n : {9, 40, 2500, 5000})
+      for (int leaf : {0, 1})
+        for (int D : {2, 3})
+          cases.push_back({std::string("spatial centre, ") + kind + " n=" + std::to_string(n) +
+                               " leaf=" + std::to_string(leaf) + " D=" + std::to_string(D),
+                           [=] { return spatial_centre_case(kind, n, D, leaf); }});
+  int fail = 0;
+  for (auto &c : cases)
+    if (only.empty() || c.name.find(only) != std::string::npos) {
+      const bool ok = c.run();
+      printf("%-66s %s\n", c.name.c_str(), ok ? "ok" : "FAILED");
+      fflush(stdout);
+      fail += !ok;
+    }
+  printf(fail ? "%d FAILED\n" : "ALL OK\n", fail);
+  return fail ? 1 : 0;
+}
