@@ -24,6 +24,7 @@
 // knn.h:566-752).
 #pragma clang fp contract(off)
 #include <new>
+#include <type_traits>
 
 #include "cukd/spatial-kdtree.h"
 #include "cukd_common.h"
@@ -811,10 +812,11 @@ __global__ __launch_bounds__(256) void k_spatial_query(const cukd_spatial_node *
   const size_t out = (size_t)qi * k;
   list.write(k, ids + out, dist2 ? dist2 + out : nullptr, ret ? ret + qi : nullptr, nullptr);
   // stack overflow: fcp reports no result, knn returns -1 (fcp.h:317-320,
-  // knn.h:620-623 print "STACK OVERFLOW" and return -1)
+  // knn.h:620-623 print "STACK OVERFLOW" and return -1) where the caller takes
+  // the radii, and leaves the row as found
   if (!ok) {
-    if (ret) ret[qi] = -1.f;
-    else ids[qi] = -1;
+    if (std::is_same<L, RegClosest>::value) ids[qi] = -1;
+    else if (ret) ret[qi] = -1.f;
   }
 }
 
@@ -861,10 +863,11 @@ __global__ __launch_bounds__(128) void k_spatial_query_any(const cukd_spatial_no
   if (stats) atomicAdd(stats, (unsigned long long)visits);
   ResultOps<R>::write(st, i, k, ids, dist2, ret, no_lists);
   // stack overflow: fcp reports no result, knn returns -1 (fcp.h:317-320,
-  // knn.h:620-623 print "STACK OVERFLOW" and return -1)
+  // knn.h:620-623 print "STACK OVERFLOW" and return -1) where the caller takes
+  // the radii, and leaves the row as found
   if (!ok) {
-    if (ret) ret[i] = -1.f;
-    else ids[i] = -1;
+    if (std::is_same<R, cukd::FCPResult>::value) ids[i] = -1;
+    else if (ret) ret[i] = -1.f;
   }
 }
 

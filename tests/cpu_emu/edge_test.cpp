@@ -120,6 +120,39 @@ bool spatial_centre_case(const char *kind, int n, int D, int leaf)
   return ok;
 }
 
+// A kNN query that overflows the reference's traversal stack, without an
+// array for the radii: every row is the oracle's, its own and the others'.
+// plain: through the kernel that trees of 2^29 nodes and more take.
+bool spatial_overflow_case(bool plain, int method, int list)
+{
+  const int n = 120, nq = 70, k = 4;
+  const cukd_layout L = floats(3);
+  const oc_layout O = ocl(L);
+  std::vector<float> pts(3 * n, 0.f), q;
+  for (int i = 0; i < n; i++) pts[3 * i] = std::ldexp(1.f, -i);
+  uint64_t seed = 5;
+  for (int i = 0; i < 3 * nq; i++) q.push_back(unit(seed));
+  for (int i = 40; i < nq; i += 9) q[3 * i] = q[3 * i + 1] = q[3 * i + 2] = 0.f;
+  const SpatialRef ref(pts, L, 1);
+  Dev<float> dp(pts), dq(q), dd((size_t)nq * k);
+  Dev<int32_t> di((size_t)nq * k);
+  cukd_spatial_tree t;
+  if (cukd_spatial_build(&t, dp.p, n, &L, 1, nullptr, nullptr) != CUKD_OK) return false;
+  const int nodes = t.num_nodes;
+  if (plain) t.num_nodes = (1 << 29) + 1;  // read for the choice of the kernel only
+  std::vector<int32_t> ri((size_t)nq * k);
+  std::vector<float> rd((size_t)nq * k), rr(nq);
+  oc_spatial_knn(method, list, k, ref.nodes.data(), ref.prims.data(), ref.box.data(), pts.data(),
+                 &O, q.data(), nq, INFINITY, ri.data(), rd.data(), rr.data(), 1);
+  bool ok = rr[49] == -1.f && rr[0] != -1.f;  // some overflow, some do not
+  ok = ok && cukd_spatial_knn(method, list, k, &t, &L, dq.p, nq, INFINITY, di.p, dd.p, nullptr,
+                              nullptr) == CUKD_OK &&
+       di.same(ri) && dd.same(rd);
+  t.num_nodes = nodes;
+  cukd_spatial_free(&t, nullptr, nullptr);
+  return ok;
+}
+
 }  // namespace
 
 int main(int argc, char **argv)
@@ -138,6 +171,11 @@ int main(int argc, char **argv)
           cases.push_back({std::string("spatial centre, ") + kind + " n=" + std::to_string(n) +
                                " leaf=" + std::to_string(leaf) + " D=" + std::to_string(D),
                            [=] { return spatial_centre_case(kind, n, D, leaf); }});
+  for (bool plain : {false, true})
+    for (int list : {CUKD_LIST_FIXED, CUKD_LIST_HEAP})
+      cases.push_back({std::string("spatial overflow without radii") + (plain ? ", plain" : "") +
+                           (list == CUKD_LIST_HEAP ? ", heap" : ""),
+                       [=] { return spatial_overflow_case(plain, CUKD_STACK_BASED, list); }});
   int fail = 0;
   for (auto &c : cases)
     if (only.empty() || c.name.find(only) != std::string::npos) {
