@@ -347,7 +347,7 @@ int cukd_compute_bounds(void *d_bounds, const void *d_points, int32_t n,
 namespace {
 
 struct TuneKey {
-  int D, trav, list, k, bucket, forest;
+  int D, trav, list, k, bucket, forest, box;
   bool operator<(const TuneKey &o) const
   {
     return memcmp(this, &o, sizeof(TuneKey)) < 0;
@@ -355,7 +355,6 @@ struct TuneKey {
 };
 struct TuneVal {
   int block, sort;
-  bool box;
 };
 std::mutex g_tune_mu;
 std::map<TuneKey, TuneVal> g_tune;
@@ -371,18 +370,21 @@ int log2_bucket(int n)
 
 // Launches the query in a (order unset).  CUKD_QUERY_SORT: Morton-ordered
 // launch.  CUKD_QUERY_AUTOTUNE: the first call per (dims, traversal, list,
-// k, log2 nq, forest) times workgroup sizes 64/128/256 with and without
-// ordering, and with and without box pruning where the kernel allows it,
-// on these very inputs (every variant writes identical results),
-// synchronising the stream once, and caches the fastest; later calls use
-// the cache.  repeatable = false (multi-round lists) only reads the cache.
+// k, log2 nq, forest, box-pruned or not) times workgroup sizes 64/128/256 with
+// and without ordering on these very inputs (every variant writes identical
+// results), synchronising the stream once, and caches the fastest; later calls
+// use the cache.  Box pruning is no choice of the tuner: it was never the
+// slower one (142 calls of 1 .. 8 dims, 50 .. 10M points, 1 .. 1M queries and
+// all lists and traversals: 0.99 .. 10 times the plain traversals' speed), and
+// whether a call may prune depends on more than its sizes.
+// repeatable = false (multi-round lists) only reads the cache.
 // order_ws (nullable): caller-owned ordering scratch of order_ws_bytes.
 static int run_queries(QueryArgs a, int D, int traversal, int flags, const MemResource &mr,
                        void *order_ws, size_t order_ws_bytes, bool repeatable,
                        hipStream_t stream, const char *what)
 {
-  TuneVal cfg{0, (flags & CUKD_QUERY_SORT) ? 1 : 0, !(flags & CUKD_QUERY_ONE_PER_LANE)};
-  const bool two_ok = box_ok(a);
+  TuneVal cfg{0, (flags & CUKD_QUERY_SORT) ? 1 : 0};
+  a.box = !(flags & CUKD_QUERY_ONE_PER_LANE);
   bool tune = false;
   TuneKey key;
   memset(&key, 0, sizeof(key));
@@ -392,6 +394,7 @@ static int run_queries(QueryArgs a, int D, int traversal, int flags, const MemRe
   key.k = a.k;
   key.bucket = log2_bucket(a.nq);
   key.forest = a.fq.seg_off != nullptr;
+  key.box = box_ok(a);
   if (flags & CUKD_QUERY_AUTOTUNE) {
     std::lock_guard<std::mutex> lk(g_tune_mu);
     auto it = g_tune.find(key);
@@ -417,13 +420,12 @@ static int run_queries(QueryArgs a, int D, int traversal, int flags, const MemRe
     float best = 3.4e38f;
     TuneVal bestv = cfg;
     const int blocks[3] = {64, 128, 256};
-    for (int box = 0; box <= (two_ok ? 1 : 0) && e == hipSuccess; box++)
     for (int sort = 0; sort < 2 && e == hipSuccess; sort++)
       for (int bi = 0; bi < 3 && e == hipSuccess; bi++) {
         QueryArgs v = a;
         v.block = blocks[bi];
-        v.box = box != 0;
-        v.stats = nullptr;  // statistics count the final launch only
+        v.box = key.box != 0;  // the final launch's kernel
+        v.stats = nullptr;     // statistics count the final launch only
         for (int rep = 0; rep < 3 && e == hipSuccess; rep++) {
           if (rep == 1) e = hipEventRecord(e0, stream);
           v.order = sort ? make_query_order(otmp, a.queries, a.nq, D, stream) : nullptr;
@@ -435,7 +437,7 @@ static int run_queries(QueryArgs a, int D, int traversal, int flags, const MemRe
         if (e == hipSuccess) e = hipEventElapsedTime(&ms, e0, e1);
         if (e == hipSuccess && ms < best) {
           best = ms;
-          bestv = TuneVal{blocks[bi], sort, box != 0};
+          bestv = TuneVal{blocks[bi], sort};
         }
       }
     if (e0) (void)hipEventDestroy(e0);
@@ -448,8 +450,6 @@ static int run_queries(QueryArgs a, int D, int traversal, int flags, const MemRe
   }
   if (e == hipSuccess) {
     a.block = cfg.block;
-    a.box = cfg.box;
-    a.presorted = (flags & CUKD_QUERY_PRESORTED) != 0;
     a.order = cfg.sort ? make_query_order(otmp, a.queries, a.nq, D, stream) : nullptr;
     e = launch_query(D, traversal, a, stream);
   }

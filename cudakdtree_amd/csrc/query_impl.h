@@ -383,7 +383,6 @@ struct QueryArgs {
   bool box = true;  // k_query_box where the call allows it
   uint64_t tree_bytes = 0;  // bytes of the tree array (forests: all trees)
   int max_n = 0;            // forests: points of the largest tree
-  bool presorted = false;   // queries already in Morton order (CUKD_QUERY_PRESORTED)
 };
 
 // persistent multi-round lists (cukd_knn_accumulate)

@@ -82,24 +82,25 @@ typedef struct cukd_mem_resource {
 #define CUKD_QUERY_SORT 1 /* Morton-order the queries before traversal
                              (results are returned in input order)      */
 #define CUKD_QUERY_AUTOTUNE 2 /* first call per (dims, traversal, list, k,
-                             log2 nq): time workgroup sizes 64/128/256 with
-                             and without Morton ordering, and one or two
-                             queries per lane where two apply, on the caller's
-                             inputs (synchronises the stream once), keep
-                             the fastest for later calls; results are the
-                             same for every choice.  Not for multi-round
+                             log2 nq, box-pruned or not): time workgroup
+                             sizes 64/128/256 with and without Morton
+                             ordering on the caller's inputs (synchronises
+                             the stream once), keep the fastest for later
+                             calls; results are the same for every choice.  Not for multi-round
                              lists (they only use an already tuned choice) */
 #define CUKD_QUERY_ONE_PER_LANE 4 /* the traversals of cukd/traverse.h as
-                             they stand, node for node.  By default queries
+                             they stand, node for node, also with
+                             CUKD_QUERY_AUTOTUNE.  By default queries
                              over a tree with round-robin split dims (and
                              under 4 GiB) also skip subtrees whose cell is
                              beyond the cull distance and keep their lists
                              in registers; results are identical either
                              way */
 #define CUKD_QUERY_PRESORTED 8 /* the queries are already in Morton order
-                             (e.g. permuted by cukd_query_order): launch
-                             with the shape of a CUKD_QUERY_SORT launch,
-                             without ordering them again */
+                             (e.g. permuted by cukd_query_order) and are
+                             not ordered again.  The launch is that of a
+                             call without flags, which suits them: their
+                             speed comes from their order */
 
 /* Builds a left-balanced k-d tree in place over d_points[0..n).
  * Replaces template<data_t,traits> buildTree / buildTree_thrust /

@@ -153,6 +153,65 @@ bool spatial_overflow_case(bool plain, int method, int list)
   return ok;
 }
 
+// launches since 'from' that name the kernel
+int launches_of(const char *kernel, size_t from)
+{
+  int c = 0;
+  for (size_t i = from; i < emu_launches.size(); i++)
+    c += emu_launches[i].find(kernel) != std::string::npos;
+  return c;
+}
+
+// An autotuned call that may not prune by box leaves nothing behind that keeps
+// a later one of the same sizes from it, and a call with
+// CUKD_QUERY_ONE_PER_LANE never prunes, whatever is cached.
+bool autotune_case(const char *first, int k)
+{
+  const int n = 700, nq = 90;
+  const bool expl = !strcmp(first, "explicit dims");
+  const cukd_layout L = floats(3), X{3, CUKD_SCALAR_F32, 20, 0, 16, 4};
+  const oc_layout O = ocl(L), OX = ocl(X);
+  uint64_t seed = 3 + k;
+  std::vector<float> pts, q, rows, box(6);
+  for (int i = 0; i < 3 * n; i++) pts.push_back(unit(seed));
+  for (int i = 0; i < 3 * nq; i++) q.push_back(unit(seed));
+  for (int i = 0; i < n; i++) {
+    rows.insert(rows.end(), pts.begin() + 3 * i, pts.begin() + 3 * i + 3);
+    rows.insert(rows.end(), 2, 0.f);
+  }
+  oc_build_host(pts.data(), n, &O, nullptr);
+  oc_build_host(rows.data(), n, &OX, box.data());
+  Dev<float> dt(pts), dx(rows), dq(q), dd((size_t)nq * k);
+  Dev<int32_t> di((size_t)nq * k);
+  std::vector<int32_t> ri((size_t)nq * k);
+  std::vector<float> rd((size_t)nq * k);
+  oc_knn(OC_STACK_BASED, OC_LIST_HEAP, k, pts.data(), n, &O, nullptr, q.data(), nq, INFINITY,
+         ri.data(), rd.data(), nullptr, nullptr, 1);
+  auto knn = [&](const float *tree, const cukd_layout &lay, float cutoff, int flags) {
+    return cukd_knn(CUKD_STACK_BASED, CUKD_LIST_HEAP, k, tree, n, &lay, nullptr, dq.p, nq, cutoff,
+                    di.p, dd.p, nullptr, CUKD_QUERY_AUTOTUNE | flags, nullptr,
+                    nullptr) == CUKD_OK;
+  };
+  Dev<unsigned long long> count(1);
+  if (!strcmp(first, "counted")) cukd_set_traversal_stats(count.p);
+  bool ok = expl ? knn(dx.p, X, INFINITY, 0)
+                 : knn(dt.p, L, !strcmp(first, "NaN cutoff") ? NAN : INFINITY,
+                       !strcmp(first, "one per lane") ? CUKD_QUERY_ONE_PER_LANE : 0);
+  cukd_set_traversal_stats(nullptr);
+  ok = ok && launches_of("k_query_box", 0) == 0;
+  // the plain call: pruned, now and once it is tuned
+  for (int rep = 0; rep < 2; rep++) {
+    const size_t from = emu_launches.size();
+    ok = ok && knn(dt.p, L, INFINITY, 0) && di.same(ri) && dd.same(rd) &&
+         launches_of("k_query_box", from) > 0 &&
+         emu_launches.back().find("k_query_box") != std::string::npos;
+  }
+  const size_t from = emu_launches.size();
+  ok = ok && knn(dt.p, L, INFINITY, CUKD_QUERY_ONE_PER_LANE) && di.same(ri) && dd.same(rd) &&
+       launches_of("k_query_box", from) == 0;
+  return ok;
+}
+
 }  // namespace
 
 int main(int argc, char **argv)
@@ -176,9 +235,15 @@ int main(int argc, char **argv)
       cases.push_back({std::string("spatial overflow without radii") + (plain ? ", plain" : "") +
                            (list == CUKD_LIST_HEAP ? ", heap" : ""),
                        [=] { return spatial_overflow_case(plain, CUKD_STACK_BASED, list); }});
+  int k = 20;
+  for (const char *first : {"counted", "NaN cutoff", "explicit dims", "one per lane"}) {
+    k++;
+    cases.push_back({std::string("autotune after ") + first, [=] { return autotune_case(first, k); }});
+  }
   int fail = 0;
   for (auto &c : cases)
     if (only.empty() || c.name.find(only) != std::string::npos) {
+      emu_launches.clear();
       const bool ok = c.run();
       printf("%-66s %s\n", c.name.c_str(), ok ? "ok" : "FAILED");
       fflush(stdout);

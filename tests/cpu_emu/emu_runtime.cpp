@@ -8,6 +8,7 @@
 
 thread_local emu_uint3 threadIdx, blockIdx;
 emu_uint3 blockDim, gridDim;
+std::vector<std::string> emu_launches;
 
 // Fiber switch for x86-64 (System V): saves the callee-saved registers on
 // the current stack, stores its stack pointer in *save_sp and continues on

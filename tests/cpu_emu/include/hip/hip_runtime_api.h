@@ -6,6 +6,9 @@
 #include <stddef.h>
 #include <stdint.h>
 
+#include <string>
+#include <vector>
+
 typedef int hipError_t;
 enum {
   hipSuccess = 0,
@@ -38,6 +41,9 @@ struct float3 { float x, y, z; };
 struct float4 { float x, y, z, w; };
 inline uint2 make_uint2(unsigned x, unsigned y) { return uint2{x, y}; }
 inline float3 make_float3(float x, float y, float z) { return float3{x, y, z}; }
+
+// the kernels launched so far, as their launches name them
+extern std::vector<std::string> emu_launches;
 
 #define HIP_SYMBOL(x) (&(x))
 
