@@ -124,7 +124,7 @@ int build_bounds_only(void *d_bounds, const void *d_points, int n, const cukd_la
                       hipStream_t s);
 
 size_t query_order_temp_bytes(int nq);
-int32_t *make_query_order(void *tmp, const float *q, int nq, int D, hipStream_t s);
+int32_t *make_query_order(hipError_t &e, void *tmp, const float *q, int nq, int D, hipStream_t s);
 
 hipError_t launch_query_1(int, const QueryArgs &, hipStream_t);
 hipError_t launch_query_2(int, const QueryArgs &, hipStream_t);
@@ -428,7 +428,7 @@ static int run_queries(QueryArgs a, int D, int traversal, int flags, const MemRe
         v.stats = nullptr;     // statistics count the final launch only
         for (int rep = 0; rep < 3 && e == hipSuccess; rep++) {
           if (rep == 1) e = hipEventRecord(e0, stream);
-          v.order = sort ? make_query_order(otmp, a.queries, a.nq, D, stream) : nullptr;
+          v.order = sort ? make_query_order(e, otmp, a.queries, a.nq, D, stream) : nullptr;
           if (e == hipSuccess) e = launch_query(D, traversal, v, stream);
         }
         if (e == hipSuccess) e = hipEventRecord(e1, stream);
@@ -450,8 +450,8 @@ static int run_queries(QueryArgs a, int D, int traversal, int flags, const MemRe
   }
   if (e == hipSuccess) {
     a.block = cfg.block;
-    a.order = cfg.sort ? make_query_order(otmp, a.queries, a.nq, D, stream) : nullptr;
-    e = launch_query(D, traversal, a, stream);
+    a.order = cfg.sort ? make_query_order(e, otmp, a.queries, a.nq, D, stream) : nullptr;
+    if (e == hipSuccess) e = launch_query(D, traversal, a, stream);
   }
   if (owned) mr.release(otmp, stream);
   if (e != hipSuccess) {
@@ -702,8 +702,8 @@ int cukd_query_order(const float *d_queries, int32_t nq, int32_t num_dims, int32
   MemResource mr{mem};
   void *tmp = nullptr;
   if (mr.alloc(&tmp, query_order_temp_bytes(nq), stream) != 0) return CUKD_ERR_ALLOC;
-  const int32_t *order = make_query_order(tmp, d_queries, nq, num_dims, stream);
-  hipError_t e = hipGetLastError();
+  hipError_t e = hipSuccess;
+  const int32_t *order = make_query_order(e, tmp, d_queries, nq, num_dims, stream);
   if (e == hipSuccess)
     e = hipMemcpyAsync(d_order, order, (size_t)nq * 4, hipMemcpyDeviceToDevice, stream);
   mr.release(tmp, stream);
@@ -812,15 +812,16 @@ static int spatial_query(int traversal, int list_kind, int k, const cukd_spatial
   a.prune = !g_stats && spatial_prunable(tree, layout->num_dims);
   a.order = nullptr;
   void *otmp = nullptr;
+  hipError_t e = hipSuccess;
   if (spatial_wants_order(a, stream)) {
     if (pool_malloc(&otmp, query_order_temp_bytes(nq), stream) == hipSuccess && otmp) {
-      a.order = make_query_order(otmp, d_queries, nq, layout->num_dims, stream);
+      a.order = make_query_order(e, otmp, d_queries, nq, layout->num_dims, stream);
     } else {
       otmp = nullptr;
       (void)hipGetLastError();  // no scratch: the queries run as given
     }
   }
-  const hipError_t e = launch_spatial_query(layout->num_dims, traversal, a, stream);
+  if (e == hipSuccess) e = launch_spatial_query(layout->num_dims, traversal, a, stream);
   if (otmp) (void)hipFreeAsync(otmp, stream);
   if (e != hipSuccess) {
     set_last_error("spatial query launch failed: %s", hipGetErrorString(e));

@@ -161,11 +161,21 @@ void set_last_error(const char *fmt, ...);
     }                                                                        \
   } while (0)
 
+// Launches a kernel unless an earlier step failed (e); e is then the launch's
+// own status, so no kernel works on what a refused launch did not write.
+#define CUKD_LAUNCH(e, ...)                                                  \
+  do {                                                                       \
+    if ((e) == hipSuccess) {                                                 \
+      hipLaunchKernelGGL(__VA_ARGS__);                                       \
+      (e) = hipGetLastError();                                               \
+    }                                                                        \
+  } while (0)
+
 // Exclusive prefix sum of n uint32 (stream-ordered, several launches);
-// 'scratch' holds at least scan_scratch_words(n) words.
+// 'scratch' holds at least scan_scratch_words(n) words.  e as in CUKD_LAUNCH.
 size_t scan_scratch_words(long long n);
-void scan_exclusive(const uint32_t *in, uint32_t *out, long long n, uint32_t *scratch,
-                    hipStream_t s);
+void scan_exclusive(hipError_t &e, const uint32_t *in, uint32_t *out, long long n,
+                    uint32_t *scratch, hipStream_t s);
 
 // Memory resource used for builder temporaries.
 void clear_last_error();

@@ -285,19 +285,19 @@ size_t query_order_temp_bytes(int nq)
 }
 
 template <int DC, int ITEMS>
-static void launch_order(int32_t *order, uint32_t *th, uint32_t *tot, const uint32_t *acc,
-                         int nblocks, const float *q, int nq, int tiles, hipStream_t s)
+static void launch_order(hipError_t &e, int32_t *order, uint32_t *th, uint32_t *tot,
+                         const uint32_t *acc, int nblocks, const float *q, int nq, int tiles, hipStream_t s)
 {
-  hipLaunchKernelGGL((k_qcount<DC, ITEMS>), dim3(tiles), dim3(QO_NT), 0, s, th, q, nq, acc, nblocks);
-  hipLaunchKernelGGL(k_qcolscan, dim3(QO_BLOCKS), dim3(QO_SCAN_NT * QO_SPLIT), 0, s, th, tot,
-                     tiles);
-  hipLaunchKernelGGL((k_qplace<DC, ITEMS>), dim3(tiles), dim3(QO_NT), 0, s, order,
-                     (const uint32_t *)th, (const uint32_t *)tot, q, nq, acc, nblocks);
+  CUKD_LAUNCH(e, (k_qcount<DC, ITEMS>), dim3(tiles), dim3(QO_NT), 0, s, th, q, nq, acc, nblocks);
+  CUKD_LAUNCH(e, k_qcolscan, dim3(QO_BLOCKS), dim3(QO_SCAN_NT * QO_SPLIT), 0, s, th, tot,
+              tiles);
+  CUKD_LAUNCH(e, (k_qplace<DC, ITEMS>), dim3(tiles), dim3(QO_NT), 0, s, order,
+              (const uint32_t *)th, (const uint32_t *)tot, q, nq, acc, nblocks);
 }
 
 // Writes the launch order of nq queries into the front of 'tmp' (which
-// holds query_order_temp_bytes(nq) bytes) and returns it.
-int32_t *make_query_order(void *tmp, const float *q, int nq, int D, hipStream_t s)
+// holds query_order_temp_bytes(nq) bytes) and returns it.  e as in CUKD_LAUNCH.
+int32_t *make_query_order(hipError_t &e, void *tmp, const float *q, int nq, int D, hipStream_t s)
 {
   uint8_t *t = (uint8_t *)tmp;
   int32_t *order = (int32_t *)t;
@@ -315,12 +315,12 @@ int32_t *make_query_order(void *tmp, const float *q, int nq, int D, hipStream_t 
   long long T = blocks * QB_NT;
   T -= T % D;
   if (T < D) T = D;  // E >= D, and blocks * QB_NT >= 256 >= D
-  hipLaunchKernelGGL(k_qbounds, dim3((unsigned)blocks), dim3(QB_NT), 0, s, acc, q, E, D, T);
-#define CUKD_QORDER_CASE(DCv)                                                                   \
-  case DCv:                                                                                     \
-    if (items == 4) launch_order<DCv, 4>(order, th, tot, acc, (int)blocks, q, nq, tiles, s);    \
-    else if (items == 8) launch_order<DCv, 8>(order, th, tot, acc, (int)blocks, q, nq, tiles, s); \
-    else launch_order<DCv, 16>(order, th, tot, acc, (int)blocks, q, nq, tiles, s);              \
+  CUKD_LAUNCH(e, k_qbounds, dim3((unsigned)blocks), dim3(QB_NT), 0, s, acc, q, E, D, T);
+#define CUKD_QORDER_CASE(DCv)                                                                      \
+  case DCv:                                                                                        \
+    if (items == 4) launch_order<DCv, 4>(e, order, th, tot, acc, (int)blocks, q, nq, tiles, s);    \
+    else if (items == 8) launch_order<DCv, 8>(e, order, th, tot, acc, (int)blocks, q, nq, tiles, s); \
+    else launch_order<DCv, 16>(e, order, th, tot, acc, (int)blocks, q, nq, tiles, s);              \
     break
   switch (D) {
     CUKD_QORDER_CASE(1);

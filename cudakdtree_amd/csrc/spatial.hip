@@ -139,17 +139,17 @@ size_t scan_scratch_words(long long n)
   return w + 1;
 }
 
-void scan_exclusive(const uint32_t *in, uint32_t *out, long long n, uint32_t *scratch,
-                    hipStream_t s)
+void scan_exclusive(hipError_t &e, const uint32_t *in, uint32_t *out, long long n,
+                    uint32_t *scratch, hipStream_t s)
 {
   if (n <= 0) return;
   const long long tiles = (n + SCAN_TILE - 1) / SCAN_TILE;
   uint32_t *sums = scratch;
-  hipLaunchKernelGGL(k_scan_tiles, dim3((unsigned)tiles), dim3(SCAN_NT), 0, s, in, out, sums, n);
+  CUKD_LAUNCH(e, k_scan_tiles, dim3((unsigned)tiles), dim3(SCAN_NT), 0, s, in, out, sums, n);
   if (tiles > 1) {
-    scan_exclusive(sums, sums, tiles, scratch + tiles + 1, s);
-    hipLaunchKernelGGL(k_scan_add, dim3((unsigned)tiles), dim3(SCAN_NT), 0, s, out,
-                       (const uint32_t *)sums, n);
+    scan_exclusive(e, sums, sums, tiles, scratch + tiles + 1, s);
+    CUKD_LAUNCH(e, k_scan_add, dim3((unsigned)tiles), dim3(SCAN_NT), 0, s, out,
+                (const uint32_t *)sums, n);
   }
 }
 
@@ -478,6 +478,7 @@ int spatial_build_impl(cukd_spatial_tree *tree, const void *d_points, int n, con
                        int leaf_threshold, hipStream_t s, const MemResource &mem)
 {
   const uint32_t thr = leaf_threshold <= 0 ? 8u : (uint32_t)leaf_threshold;
+  (void)hipGetLastError();  // an earlier call's error is no launch's below
   if (n > 0) {
     const uint8_t *pts = (const uint8_t *)d_points;
     bool deep = false;
@@ -530,12 +531,12 @@ static int spatial_build_rounds(cukd_spatial_tree *tree, const void *d_points, i
   int rc = CUKD_OK;
   hipError_t e = hipSuccess;
 
-  hipLaunchKernelGGL(k_sp_init, dim3((unsigned)((nn + 255) / 256)), dim3(256), 0, s, nodes, pp[0],
-                     pn[0], degen, n, D);
+  CUKD_LAUNCH(e, k_sp_init, dim3((unsigned)((nn + 255) / 256)), dim3(256), 0, s, nodes, pp[0],
+              pn[0], degen, n, D);
   if (n > 0) {
     int blocks = (n + 255) / 256;
     if (blocks > 2048) blocks = 2048;
-    hipLaunchKernelGGL(k_sp_root_bounds, dim3(blocks), dim3(256), 0, s, nodes, pts, n, L);
+    CUKD_LAUNCH(e, k_sp_root_bounds, dim3(blocks), dim3(256), 0, s, nodes, pts, n, L);
   }
   // open nodes [a, b); node 1 is the reference's reserved empty leaf, so
   // the first children are numbered from 2
@@ -545,24 +546,24 @@ static int spatial_build_rounds(cukd_spatial_tree *tree, const void *d_points, i
     levels++;
     const int cnt = b - a;
     const int g = (cnt + 255) / 256;
-    hipLaunchKernelGGL(k_sp_decide, dim3(g), dim3(256), 0, s, nodes, nflag, degen, a, b, D,
-                       thr);
-    scan_exclusive(nflag, nexcl, cnt, scratch, s);
-    hipLaunchKernelGGL(k_sp_alloc, dim3(g), dim3(256), 0, s, nodes, (const uint32_t *)nexcl, a, b, next,
-                       D);
+    CUKD_LAUNCH(e, k_sp_decide, dim3(g), dim3(256), 0, s, nodes, nflag, degen, a, b, D,
+                thr);
+    scan_exclusive(e, nflag, nexcl, cnt, scratch, s);
+    CUKD_LAUNCH(e, k_sp_alloc, dim3(g), dim3(256), 0, s, nodes, (const uint32_t *)nexcl, a, b, next,
+                D);
     if (n > 0) {
-      hipLaunchKernelGGL(k_sp_classify, dim3(gp), dim3(256), 0, s, (const SpNode *)nodes,
-                         (const uint32_t *)pp[cur], (const uint32_t *)pn[cur], pflag, pts, n, L);
-      scan_exclusive(pflag, pexcl, n, scratch, s);
-      hipLaunchKernelGGL(k_sp_scatter, dim3(gp), dim3(256), 0, s, nodes, (const uint32_t *)pp[cur],
-                         (const uint32_t *)pn[cur], (const uint32_t *)pflag, (const uint32_t *)pexcl,
-                         pp[cur ^ 1], pn[cur ^ 1], pts, n, L);
+      CUKD_LAUNCH(e, k_sp_classify, dim3(gp), dim3(256), 0, s, (const SpNode *)nodes,
+                  (const uint32_t *)pp[cur], (const uint32_t *)pn[cur], pflag, pts, n, L);
+      scan_exclusive(e, pflag, pexcl, n, scratch, s);
+      CUKD_LAUNCH(e, k_sp_scatter, dim3(gp), dim3(256), 0, s, nodes, (const uint32_t *)pp[cur],
+                  (const uint32_t *)pn[cur], (const uint32_t *)pflag, (const uint32_t *)pexcl,
+                  pp[cur ^ 1], pn[cur ^ 1], pts, n, L);
       cur ^= 1;
     }
-    hipLaunchKernelGGL(k_sp_close, dim3(g), dim3(256), 0, s, nodes, (const uint32_t *)nflag,
-                       (const uint32_t *)nexcl, a, b, num_split);
+    CUKD_LAUNCH(e, k_sp_close, dim3(g), dim3(256), 0, s, nodes, (const uint32_t *)nflag,
+                (const uint32_t *)nexcl, a, b, num_split);
     uint32_t h_split = 0;
-    e = hipMemcpyAsync(&h_split, num_split, 4, hipMemcpyDeviceToHost, s);
+    if (e == hipSuccess) e = hipMemcpyAsync(&h_split, num_split, 4, hipMemcpyDeviceToHost, s);
     if (e == hipSuccess) e = hipStreamSynchronize(s);
     if (e != hipSuccess) break;
     a = next;
@@ -578,19 +579,19 @@ static int spatial_build_rounds(cukd_spatial_tree *tree, const void *d_points, i
       rc = CUKD_ERR_ALLOC;
     } else {
       const int g = (num_nodes + 255) / 256;
-      hipLaunchKernelGGL(k_sp_leaf_counts, dim3(g), dim3(256), 0, s, (const SpNode *)nodes, nflag,
-                         num_nodes);
-      scan_exclusive(nflag, nexcl, num_nodes, scratch, s);
+      CUKD_LAUNCH(e, k_sp_leaf_counts, dim3(g), dim3(256), 0, s, (const SpNode *)nodes, nflag,
+                  num_nodes);
+      scan_exclusive(e, nflag, nexcl, num_nodes, scratch, s);
       if (n > 0)
-        hipLaunchKernelGGL(k_sp_write_prims, dim3(gp), dim3(256), 0, s, (const SpNode *)nodes,
-                           (const uint32_t *)nexcl, (const uint32_t *)pp[cur],
-                           (const uint32_t *)pn[cur], out_prims, n);
-      hipLaunchKernelGGL(k_sp_write_nodes, dim3(g), dim3(256), 0, s, (const SpNode *)nodes,
-                         (const uint32_t *)nexcl, out_nodes, num_nodes, isf);
-      hipLaunchKernelGGL(k_sp_bounds_out, dim3(1), dim3(64), 0, s, (const SpNode *)nodes,
-                         bounds_dev, D, isf);
+        CUKD_LAUNCH(e, k_sp_write_prims, dim3(gp), dim3(256), 0, s, (const SpNode *)nodes,
+                    (const uint32_t *)nexcl, (const uint32_t *)pp[cur],
+                    (const uint32_t *)pn[cur], out_prims, n);
+      CUKD_LAUNCH(e, k_sp_write_nodes, dim3(g), dim3(256), 0, s, (const SpNode *)nodes,
+                  (const uint32_t *)nexcl, out_nodes, num_nodes, isf);
+      CUKD_LAUNCH(e, k_sp_bounds_out, dim3(1), dim3(64), 0, s, (const SpNode *)nodes,
+                  bounds_dev, D, isf);
       uint32_t hb[2 * CUKD_MAX_DIMS + 1];
-      e = hipMemcpyAsync(hb, bounds_dev, 4 * (2 * D + 1), hipMemcpyDeviceToHost, s);
+      if (e == hipSuccess) e = hipMemcpyAsync(hb, bounds_dev, 4 * (2 * D + 1), hipMemcpyDeviceToHost, s);
       if (e == hipSuccess) e = hipStreamSynchronize(s);
       if (e == hipSuccess) {
         for (int i = 0; i < 2 * CUKD_MAX_DIMS; i++) tree->ibounds[i] = i < 2 * D ? (int32_t)hb[i] : 0;

@@ -813,32 +813,35 @@ static int spatial_build_items(cukd_spatial_tree *tree, const uint8_t *pts, int 
   const uint32_t small = thr > (uint32_t)SPB_T ? thr : (uint32_t)SPB_T;
   const bool isf = L.scalar_type == CUKD_SCALAR_F32;
   const int gn = (n + 255) / 256;
+  // more dynamic LDS than a kernel may take unasked
+  hipError_t e = hipFuncSetAttribute((const void *)k_spb_small<D>,
+                                     hipFuncAttributeMaxDynamicSharedMemorySize,
+                                     (int)spb_lds(D, thr));
 
-  hipLaunchKernelGGL(k_spb_init, dim3(gn), dim3(256), 0, s, nodes, boxes, st, pp0, pn0,
-                     n, D);
-  hipLaunchKernelGGL(k_spb_root, dim3(gn < 512 ? gn : 512), dim3(SPB_NT), 0, s, boxes, pts, n, L);
+  CUKD_LAUNCH(e, k_spb_init, dim3(gn), dim3(256), 0, s, nodes, boxes, st, pp0, pn0,
+              n, D);
+  CUKD_LAUNCH(e, k_spb_root, dim3(gn < 512 ? gn : 512), dim3(SPB_NT), 0, s, boxes, pts, n, L);
   // Halving n points down to SPB_T takes log2(n / SPB_T) rounds where the
   // points are even, and one more to see that nothing is open; more are
   // launched, two at a time, while nodes remain.
   int rounds = 1;
   while (((long long)SPB_T << (rounds - 1)) < (long long)n && rounds < SPB_LEVELS) rounds++;
   SpRounds h;
-  hipError_t e = hipSuccess;
   for (;;) {
     for (int i = 0; i < rounds; i++) {
-      hipLaunchKernelGGL(k_spb_level, dim3(1), dim3(SPB_LNT), 0, s, nodes, boxes, st, D,
-                         small);
+      CUKD_LAUNCH(e, k_spb_level, dim3(1), dim3(SPB_LNT), 0, s, nodes, boxes, st, D,
+                  small);
       if ((uint32_t)n <= small) break;
-      hipLaunchKernelGGL(k_spb_flags<false>, dim3(tiles), dim3(SPB_NT), 0, s, (const SpNode *)nodes,
-                         (const SpRounds *)st, (const uint32_t *)pp0, (const uint32_t *)pp1,
-                         (const uint32_t *)pn0, (const uint32_t *)pn1, loc, tile, pts, n, L);
-      hipLaunchKernelGGL(k_spb_scan<false>, dim3(1), dim3(SPB_LNT), 0, s, nodes,
-                         (const SpRounds *)st, tile, (const uint16_t *)loc, tiles, n);
-      hipLaunchKernelGGL(k_spb_scatter<D>, dim3(tiles), dim3(SPB_NT), 0, s,
-                         (const SpNode *)nodes, boxes, (const SpRounds *)st, pp0, pp1, pn0, pn1,
-                         (const uint16_t *)loc, (const uint32_t *)tile, pts, n, L);
+      CUKD_LAUNCH(e, k_spb_flags<false>, dim3(tiles), dim3(SPB_NT), 0, s, (const SpNode *)nodes,
+                  (const SpRounds *)st, (const uint32_t *)pp0, (const uint32_t *)pp1,
+                  (const uint32_t *)pn0, (const uint32_t *)pn1, loc, tile, pts, n, L);
+      CUKD_LAUNCH(e, k_spb_scan<false>, dim3(1), dim3(SPB_LNT), 0, s, nodes,
+                  (const SpRounds *)st, tile, (const uint16_t *)loc, tiles, n);
+      CUKD_LAUNCH(e, k_spb_scatter<D>, dim3(tiles), dim3(SPB_NT), 0, s,
+                  (const SpNode *)nodes, boxes, (const SpRounds *)st, pp0, pp1, pn0, pn1,
+                  (const uint16_t *)loc, (const uint32_t *)tile, pts, n, L);
     }
-    e = hipMemcpyAsync(&h, st, sizeof(h), hipMemcpyDeviceToHost, s);
+    if (e == hipSuccess) e = hipMemcpyAsync(&h, st, sizeof(h), hipMemcpyDeviceToHost, s);
     if (e == hipSuccess) e = hipStreamSynchronize(s);
     if (e != hipSuccess || h.deep || h.a >= h.b) break;
     rounds = 2;
@@ -854,23 +857,24 @@ static int spatial_build_items(cukd_spatial_tree *tree, const uint8_t *pts, int 
     const int ni = h.nitems, gl = (h.next + SPB_NT - 1) / SPB_NT;
     if (mem.alloc((void **)&M, (size_t)SPB_LEVELS * ni * 4, s) != 0) rc = CUKD_ERR_ALLOC;
     if (rc == CUKD_OK) {
-      hipLaunchKernelGGL(k_spb_flags<true>, dim3(tiles), dim3(SPB_NT), 0, s, (const SpNode *)nodes,
-                         (const SpRounds *)st, (const uint32_t *)pp0, (const uint32_t *)pp1,
-                         (const uint32_t *)pn0, (const uint32_t *)pn1, loc, tile, pts, n, L);
-      hipLaunchKernelGGL(k_spb_scan<true>, dim3(1), dim3(SPB_LNT), 0, s, nodes,
-                         (const SpRounds *)st, tile, (const uint16_t *)loc, tiles, n);
-      hipLaunchKernelGGL(k_spb_items, dim3(gn), dim3(256), 0, s, (const SpRounds *)st,
-                         (const uint32_t *)pn0, (const uint32_t *)pn1, (const uint16_t *)loc,
-                         (const uint32_t *)tile, items, rank_at, n);
-      hipLaunchKernelGGL(k_spb_small<D>, dim3(ni), dim3(SPB_SNT), spb_lds(D, thr), s,
-                         (const SpNode *)nodes, st, (const uint32_t *)items, pp0, pp1, pts, L, thr,
-                         recs, pos_rec, M, ni);
-      hipLaunchKernelGGL(k_spb_large, dim3(gl), dim3(SPB_NT), 0, s, (const SpNode *)nodes,
-                         (const SpRounds *)st, (const uint32_t *)rank_at, M, ni);
-      hipLaunchKernelGGL(k_sp_bounds_out, dim3(1), dim3(64), 0, s, (const SpNode *)nodes,
-                         out_words + SPB_LEVELS, D, isf);
-      hipLaunchKernelGGL(k_spb_number, dim3(SPB_LEVELS), dim3(SPB_LNT), 0, s, M, out_words, ni);
-      e = hipMemcpyAsync(hw, out_words, 4 * (SPB_LEVELS + 2 * D), hipMemcpyDeviceToHost, s);
+      CUKD_LAUNCH(e, k_spb_flags<true>, dim3(tiles), dim3(SPB_NT), 0, s, (const SpNode *)nodes,
+                  (const SpRounds *)st, (const uint32_t *)pp0, (const uint32_t *)pp1,
+                  (const uint32_t *)pn0, (const uint32_t *)pn1, loc, tile, pts, n, L);
+      CUKD_LAUNCH(e, k_spb_scan<true>, dim3(1), dim3(SPB_LNT), 0, s, nodes,
+                  (const SpRounds *)st, tile, (const uint16_t *)loc, tiles, n);
+      CUKD_LAUNCH(e, k_spb_items, dim3(gn), dim3(256), 0, s, (const SpRounds *)st,
+                  (const uint32_t *)pn0, (const uint32_t *)pn1, (const uint16_t *)loc,
+                  (const uint32_t *)tile, items, rank_at, n);
+      CUKD_LAUNCH(e, k_spb_small<D>, dim3(ni), dim3(SPB_SNT), spb_lds(D, thr), s,
+                  (const SpNode *)nodes, st, (const uint32_t *)items, pp0, pp1, pts, L, thr,
+                  recs, pos_rec, M, ni);
+      CUKD_LAUNCH(e, k_spb_large, dim3(gl), dim3(SPB_NT), 0, s, (const SpNode *)nodes,
+                  (const SpRounds *)st, (const uint32_t *)rank_at, M, ni);
+      CUKD_LAUNCH(e, k_sp_bounds_out, dim3(1), dim3(64), 0, s, (const SpNode *)nodes,
+                  out_words + SPB_LEVELS, D, isf);
+      CUKD_LAUNCH(e, k_spb_number, dim3(SPB_LEVELS), dim3(SPB_LNT), 0, s, M, out_words, ni);
+      if (e == hipSuccess)
+        e = hipMemcpyAsync(hw, out_words, 4 * (SPB_LEVELS + 2 * D), hipMemcpyDeviceToHost, s);
       if (e == hipSuccess) e = hipMemcpyAsync(&h, st, sizeof(h), hipMemcpyDeviceToHost, s);
       if (e == hipSuccess) e = hipStreamSynchronize(s);
       *deep = e == hipSuccess && h.deep;
@@ -889,20 +893,20 @@ static int spatial_build_items(cukd_spatial_tree *tree, const uint8_t *pts, int 
       }
     }
     if (rc == CUKD_OK && e == hipSuccess && !*deep) {
-      hipLaunchKernelGGL(k_spb_ids<false>, dim3(ni + gl), dim3(SPB_NT), 0, s, (const SpNode *)nodes,
-                         (const SpRounds *)st, (const uint32_t *)items, (const uint32_t *)rank_at,
-                         (const SpRec *)recs, (const uint32_t *)M, lb, ni, rec_id, leaf_cnt,
-                         (const uint32_t *)leaf_off, out_nodes, isf);
-      scan_exclusive(leaf_cnt, leaf_off, num_nodes, scratch, s);
-      hipLaunchKernelGGL(k_spb_ids<true>, dim3(ni + gl), dim3(SPB_NT), 0, s, (const SpNode *)nodes,
-                         (const SpRounds *)st, (const uint32_t *)items, (const uint32_t *)rank_at,
-                         (const SpRec *)recs, (const uint32_t *)M, lb, ni, rec_id, leaf_cnt,
-                         (const uint32_t *)leaf_off, out_nodes, isf);
-      hipLaunchKernelGGL(k_spb_prims, dim3(gn), dim3(256), 0, s, (const SpRounds *)st,
-                         (const SpRec *)recs, (const uint32_t *)pos_rec, (const uint32_t *)rec_id,
-                         (const uint32_t *)leaf_off, (const uint32_t *)pp0, (const uint32_t *)pp1,
-                         out_prims, n);
-      e = hipStreamSynchronize(s);
+      CUKD_LAUNCH(e, k_spb_ids<false>, dim3(ni + gl), dim3(SPB_NT), 0, s, (const SpNode *)nodes,
+                  (const SpRounds *)st, (const uint32_t *)items, (const uint32_t *)rank_at,
+                  (const SpRec *)recs, (const uint32_t *)M, lb, ni, rec_id, leaf_cnt,
+                  (const uint32_t *)leaf_off, out_nodes, isf);
+      scan_exclusive(e, leaf_cnt, leaf_off, num_nodes, scratch, s);
+      CUKD_LAUNCH(e, k_spb_ids<true>, dim3(ni + gl), dim3(SPB_NT), 0, s, (const SpNode *)nodes,
+                  (const SpRounds *)st, (const uint32_t *)items, (const uint32_t *)rank_at,
+                  (const SpRec *)recs, (const uint32_t *)M, lb, ni, rec_id, leaf_cnt,
+                  (const uint32_t *)leaf_off, out_nodes, isf);
+      CUKD_LAUNCH(e, k_spb_prims, dim3(gn), dim3(256), 0, s, (const SpRounds *)st,
+                  (const SpRec *)recs, (const uint32_t *)pos_rec, (const uint32_t *)rec_id,
+                  (const uint32_t *)leaf_off, (const uint32_t *)pp0, (const uint32_t *)pp1,
+                  out_prims, n);
+      if (e == hipSuccess) e = hipStreamSynchronize(s);
     }
   }
   mem.release(M, s);

@@ -212,6 +212,69 @@ bool autotune_case(const char *first, int k)
   return ok;
 }
 
+// Runs 'call' again and again, with its first launch refused, then its second,
+// ..., until it runs through: each refusal is its error, and no launch of the
+// call works on what a refused one did not write.  'done' follows a success.
+bool refusals_reported(const std::function<int()> &call, const std::function<bool()> &done)
+{
+  for (int i = 0;; i++) {
+    emu_refuse_in = i;
+    const int rc = call();
+    const bool refused = emu_refuse_in < 0;
+    emu_refuse_in = -1;
+    if (!refused) return i > 0 && rc == CUKD_OK && done();
+    if (rc != CUKD_ERR_HIP || hipGetLastError() != hipSuccess) {
+      printf("  launch %d: rc %d\n", i, rc);
+      return false;
+    }
+  }
+}
+
+// deep: points that peel off one by one, more than the level table holds
+bool refused_spatial_build_case(int n, int D, bool deep)
+{
+  const cukd_layout L = floats(D);
+  uint64_t seed = 9;
+  std::vector<float> pts((size_t)n * D, 0.f);
+  for (int i = 0; i < n * D; i++)
+    pts[i] = !deep ? unit(seed) : i % D ? 0.f : std::ldexp(1.f, -(i / D));
+  const int leaf = deep ? 1 : 0;
+  const SpatialRef ref(pts, L, leaf);
+  Dev<float> dp(pts);
+  cukd_spatial_tree t;
+  return refusals_reported(
+      [&] { return cukd_spatial_build(&t, dp.p, n, &L, leaf, nullptr, nullptr); },
+      [&] {
+        const bool ok = ref.same(t);
+        cukd_spatial_free(&t, nullptr, nullptr);
+        return ok;
+      });
+}
+
+bool refused_sorted_query_case()
+{
+  const int n = 500, nq = 100, k = 4;
+  const cukd_layout L = floats(3);
+  const oc_layout O = ocl(L);
+  uint64_t seed = 9;
+  std::vector<float> pts, q;
+  for (int i = 0; i < 3 * n; i++) pts.push_back(unit(seed));
+  for (int i = 0; i < 3 * nq; i++) q.push_back(unit(seed));
+  oc_build_host(pts.data(), n, &O, nullptr);
+  Dev<float> dt(pts), dq(q), dd((size_t)nq * k);
+  Dev<int32_t> di((size_t)nq * k);
+  std::vector<int32_t> ri((size_t)nq * k);
+  std::vector<float> rd((size_t)nq * k);
+  oc_knn(OC_STACK_BASED, OC_LIST_FIXED, k, pts.data(), n, &O, nullptr, q.data(), nq, INFINITY,
+         ri.data(), rd.data(), nullptr, nullptr, 1);
+  return refusals_reported(
+      [&] {
+        return cukd_knn(CUKD_STACK_BASED, CUKD_LIST_FIXED, k, dt.p, n, &L, nullptr, dq.p, nq,
+                        INFINITY, di.p, dd.p, nullptr, CUKD_QUERY_SORT, nullptr, nullptr);
+      },
+      [&] { return di.same(ri) && dd.same(rd); });
+}
+
 }  // namespace
 
 int main(int argc, char **argv)
@@ -240,6 +303,10 @@ int main(int argc, char **argv)
     k++;
     cases.push_back({std::string("autotune after ") + first, [=] { return autotune_case(first, k); }});
   }
+  cases.push_back({"refused launch, spatial build", [] { return refused_spatial_build_case(5000, 3, false); }});
+  cases.push_back({"refused launch, spatial build of one leaf", [] { return refused_spatial_build_case(5, 3, false); }});
+  cases.push_back({"refused launch, deep spatial build", [] { return refused_spatial_build_case(110, 2, true); }});
+  cases.push_back({"refused launch, sorted query", [] { return refused_sorted_query_case(); }});
   int fail = 0;
   for (auto &c : cases)
     if (only.empty() || c.name.find(only) != std::string::npos) {

@@ -9,6 +9,18 @@
 thread_local emu_uint3 threadIdx, blockIdx;
 emu_uint3 blockDim, gridDim;
 std::vector<std::string> emu_launches;
+int emu_refuse_in = -1;
+static thread_local hipError_t emu_last_error = hipSuccess;
+
+bool emu_admit(const char *kernel)
+{
+  if (emu_refuse_in >= 0 && emu_refuse_in-- == 0) {
+    emu_last_error = hipErrorInvalidValue;
+    return false;
+  }
+  emu_launches.push_back(kernel);
+  return true;
+}
 
 // Fiber switch for x86-64 (System V): saves the callee-saved registers on
 // the current stack, stores its stack pointer in *save_sp and continues on
@@ -257,7 +269,12 @@ void *emu_dynamic_lds() { return emu::g_run->dyn; }
 
 // ---- runtime API ----
 const char *hipGetErrorString(hipError_t e) { return e == hipSuccess ? "no error" : "emulated error"; }
-hipError_t hipGetLastError(void) { return hipSuccess; }
+hipError_t hipGetLastError(void)
+{
+  const hipError_t e = emu_last_error;
+  emu_last_error = hipSuccess;
+  return e;
+}
 hipError_t hipMalloc(void **p, size_t n)
 {
   *p = aligned_alloc(256, (n + 255) / 256 * 256 + 256);

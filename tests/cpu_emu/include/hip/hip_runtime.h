@@ -82,7 +82,7 @@ inline void launch(void (*k)(P...), dim3 grid, dim3 block, size_t lds, A &&...ar
 }  // namespace emu
 
 #define hipLaunchKernelGGL(k, grid, block, lds, stream, ...) \
-  emu_launches.push_back(#k), emu::launch(k, dim3(grid), dim3(block), (size_t)(lds), ##__VA_ARGS__)
+  emu_admit(#k) ? emu::launch(k, dim3(grid), dim3(block), (size_t)(lds), ##__VA_ARGS__) : (void)0
 
 inline void __syncthreads() { emu::sync_point(emu::OP_BARRIER, 0, 0); }
 inline void __builtin_amdgcn_wave_barrier() { emu::sync_point(emu::OP_WAVE_BARRIER, 0, 0); }

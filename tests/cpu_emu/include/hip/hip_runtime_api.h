@@ -44,6 +44,10 @@ inline float3 make_float3(float x, float y, float z) { return float3{x, y, z}; }
 
 // the kernels launched so far, as their launches name them
 extern std::vector<std::string> emu_launches;
+// launches until one is refused, as a launch that the device cannot take is
+// (it does not run, and hipGetLastError reports it); negative: none is
+extern int emu_refuse_in;
+bool emu_admit(const char *kernel);
 
 #define HIP_SYMBOL(x) (&(x))
 
