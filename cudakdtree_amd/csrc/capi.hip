@@ -27,45 +27,56 @@ void set_last_error(const char *fmt, ...)
 
 // The library's temporaries come from a memory pool of its own, one per
 // device, that keeps up to POOL_KEEP_BYTES of freed memory across
-// synchronisations; the device's default pool keeps none, and mapping the
+// synchronisations; a device's default pool keeps none, and mapping the
 // pages again cost 0.04 .. 0.3 ms a call (10M build 4.31 -> 4.00
 // ms, 1.5M payload 1.51 -> 1.23, 1M spatial 1.45 -> 1.10).  What is
 // above the bound goes back at the next synchronisation, the rest with
 // cukd_release_memory or the process.  The pool orders reuse between streams.
-#ifdef HIP_VERSION  // a runtime with memory pools
 static constexpr uint64_t POOL_KEEP_BYTES = (uint64_t)1 << 30;
 static std::mutex g_pool_mu;
 static std::map<int, hipMemPool_t> g_pools;
 
-static hipError_t pool_malloc(void **p, size_t bytes, hipStream_t s)
+// The library's pool on the device of stream s, which need not be the current
+// device.  Null, for that device's current pool, where the program has set a
+// pool of its own or lets the default one keep memory (its choice governs),
+// while s is being captured, and where the runtime has no answer.
+static hipMemPool_t library_pool(hipStream_t s)
 {
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-  int dev = 0;
-  hipError_t e = hipStreamIsCapturing(s, &st);
-  if (e != hipSuccess) return e;
-  if (st != hipStreamCaptureStatusNone) return hipMallocAsync(p, bytes, s);
-  if ((e = hipGetDevice(&dev)) != hipSuccess) return e;
-  hipMemPool_t pool = nullptr;
-  {
-    std::lock_guard<std::mutex> lk(g_pool_mu);
-    auto it = g_pools.find(dev);
-    if (it == g_pools.end()) {
-      hipMemPoolProps props;
-      memset(&props, 0, sizeof(props));
-      props.allocType = hipMemAllocationTypePinned;
-      props.location.type = hipMemLocationTypeDevice;
-      props.location.id = dev;
-      uint64_t keep = POOL_KEEP_BYTES;
-      if (hipMemPoolCreate(&pool, &props) != hipSuccess) pool = nullptr;
-      if (pool && hipMemPoolSetAttribute(pool, hipMemPoolAttrReleaseThreshold, &keep) != hipSuccess) {
-        (void)hipMemPoolDestroy(pool);
-        pool = nullptr;
-      }
-      if (!pool) (void)hipGetLastError();  // the default pool serves
-      it = g_pools.emplace(dev, pool).first;
-    }
-    pool = it->second;
+  hipDevice_t dev = 0;
+  hipMemPool_t def = nullptr, current = nullptr, pool = nullptr;
+  uint64_t keep = 0;
+  if (hipStreamIsCapturing(s, &st) != hipSuccess || hipStreamGetDevice(s, &dev) != hipSuccess ||
+      hipDeviceGetDefaultMemPool(&def, dev) != hipSuccess ||
+      hipDeviceGetMemPool(&current, dev) != hipSuccess ||
+      hipMemPoolGetAttribute(def, hipMemPoolAttrReleaseThreshold, &keep) != hipSuccess) {
+    (void)hipGetLastError();
+    return nullptr;
   }
+  if (st != hipStreamCaptureStatusNone || current != def || keep != 0) return nullptr;
+  std::lock_guard<std::mutex> lk(g_pool_mu);
+  auto it = g_pools.find(dev);
+  if (it == g_pools.end()) {
+    hipMemPoolProps props;
+    memset(&props, 0, sizeof(props));
+    props.allocType = hipMemAllocationTypePinned;
+    props.location.type = hipMemLocationTypeDevice;
+    props.location.id = dev;
+    keep = POOL_KEEP_BYTES;
+    if (hipMemPoolCreate(&pool, &props) != hipSuccess) pool = nullptr;
+    if (pool && hipMemPoolSetAttribute(pool, hipMemPoolAttrReleaseThreshold, &keep) != hipSuccess) {
+      (void)hipMemPoolDestroy(pool);
+      pool = nullptr;
+    }
+    if (!pool) (void)hipGetLastError();  // the current pool serves
+    it = g_pools.emplace(dev, pool).first;
+  }
+  return it->second;
+}
+
+static hipError_t pool_malloc(void **p, size_t bytes, hipStream_t s)
+{
+  const hipMemPool_t pool = library_pool(s);
   return pool ? hipMallocFromPoolAsync(p, bytes, pool, s) : hipMallocAsync(p, bytes, s);
 }
 
@@ -77,13 +88,6 @@ static hipError_t pool_trim()
     if (it.second && e == hipSuccess) e = hipMemPoolTrimTo(it.second, 0);
   return e;
 }
-#else
-static hipError_t pool_malloc(void **p, size_t bytes, hipStream_t s)
-{
-  return hipMallocAsync(p, bytes, s);
-}
-static hipError_t pool_trim() { return hipSuccess; }
-#endif
 
 int MemResource::alloc(void **p, size_t bytes, hipStream_t s) const
 {

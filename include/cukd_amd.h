@@ -414,7 +414,11 @@ int cukd_set_traversal_stats(unsigned long long *d_counter);
 /* Gives back the freed device memory that the library keeps for its next
  * temporaries (up to 1 GiB per device, calls without a memory resource).
  * Memory still in use, or freed on a stream that has not got there yet,
- * stays. */
+ * stays.  Nothing is kept on a device whose current memory pool is not its
+ * default one (hipDeviceSetMemPool), or whose default pool has a release
+ * threshold: such calls take their memory from the device's current pool.
+ * The pools, like every object of this library, do not outlive
+ * hipDeviceReset: no call without a memory resource may follow it. */
 int cukd_release_memory(void);
 
 /* Message of the last failed call on this thread ("" if none). */

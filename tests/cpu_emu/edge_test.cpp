@@ -275,6 +275,41 @@ bool refused_sorted_query_case()
       [&] { return di.same(ri) && dd.same(rd); });
 }
 
+// Temporaries come from memory of the stream's device, and from the pool that
+// the program chose for it where it chose one.
+bool pool_case(const char *what)
+{
+  const int n = 600;
+  const cukd_layout L = floats(3);
+  uint64_t seed = 21;
+  std::vector<float> pts;
+  for (int i = 0; i < 3 * n; i++) pts.push_back(unit(seed));
+  Dev<float> dp(pts);
+  const bool other = !strcmp(what, "stream of another device");
+  const int dev = other ? 1 : 0;
+  hipSetDevice(dev);
+  hipStream_t s = nullptr;
+  hipStreamCreateWithFlags(&s, hipStreamNonBlocking);
+  hipSetDevice(0);
+  hipMemPool_t def = nullptr, own = nullptr;
+  hipDeviceGetDefaultMemPool(&def, dev);
+  const hipMemPoolProps props{hipMemAllocationTypePinned, {hipMemLocationTypeDevice, dev}};
+  hipMemPoolCreate(&own, &props);
+  uint64_t keep = 1 << 20, none = 0;
+  if (!strcmp(what, "a current pool")) hipDeviceSetMemPool(dev, own);
+  if (!strcmp(what, "a default pool that keeps")) hipMemPoolSetAttribute(def, hipMemPoolAttrReleaseThreshold, &keep);
+  emu_last_pool = nullptr;
+  bool ok = cukd_build_tree(dp.p, n, &L, CUKD_BUILDER_ID_DEFAULT, nullptr, s, nullptr) == CUKD_OK;
+  ok = ok && emu_last_pool && emu_last_pool->device == dev;
+  if (!strcmp(what, "a current pool")) ok = ok && emu_last_pool == own;
+  else if (!strcmp(what, "a default pool that keeps")) ok = ok && emu_last_pool == def;
+  else ok = ok && emu_last_pool != def && emu_last_pool->threshold > 0;  // the library's
+  hipDeviceSetMemPool(dev, def);
+  hipMemPoolSetAttribute(def, hipMemPoolAttrReleaseThreshold, &none);
+  hipStreamDestroy(s);
+  return ok;
+}
+
 }  // namespace
 
 int main(int argc, char **argv)
@@ -307,6 +342,9 @@ int main(int argc, char **argv)
   cases.push_back({"refused launch, spatial build of one leaf", [] { return refused_spatial_build_case(5, 3, false); }});
   cases.push_back({"refused launch, deep spatial build", [] { return refused_spatial_build_case(110, 2, true); }});
   cases.push_back({"refused launch, sorted query", [] { return refused_sorted_query_case(); }});
+  for (const char *what : {"nothing chosen", "stream of another device", "a current pool",
+                           "a default pool that keeps", "nothing chosen"})
+    cases.push_back({std::string("memory pool, ") + what, [=] { return pool_case(what); }});
   int fail = 0;
   for (auto &c : cases)
     if (only.empty() || c.name.find(only) != std::string::npos) {

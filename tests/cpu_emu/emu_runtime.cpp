@@ -5,6 +5,7 @@
 
 #include <chrono>
 #include <cstdlib>
+#include <memory>
 
 thread_local emu_uint3 threadIdx, blockIdx;
 emu_uint3 blockDim, gridDim;
@@ -280,7 +281,6 @@ hipError_t hipMalloc(void **p, size_t n)
   *p = aligned_alloc(256, (n + 255) / 256 * 256 + 256);
   return *p ? hipSuccess : hipErrorOutOfMemory;
 }
-hipError_t hipMallocAsync(void **p, size_t n, hipStream_t) { return hipMalloc(p, n); }
 hipError_t hipMallocManaged(void **p, size_t n, unsigned) { return hipMalloc(p, n); }
 hipError_t hipHostMalloc(void **p, size_t n, unsigned) { return hipMalloc(p, n); }
 hipError_t hipFree(void *p) { free(p); return hipSuccess; }
@@ -299,8 +299,6 @@ hipError_t hipMemcpyToSymbol(const void *sym, const void *src, size_t n, size_t 
 }
 hipError_t hipGetSymbolAddress(void **p, const void *sym) { *p = (void *)sym; return hipSuccess; }
 hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
-hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned) { *s = (hipStream_t)new int(0); return hipSuccess; }
-hipError_t hipStreamDestroy(hipStream_t s) { delete (int *)s; return hipSuccess; }
 hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned) { return hipSuccess; }
 hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus *st) { *st = hipStreamCaptureStatusNone; return hipSuccess; }
 hipError_t hipDeviceSynchronize(void) { return hipSuccess; }
@@ -315,6 +313,50 @@ hipError_t hipEventElapsedTime(float *ms, hipEvent_t a, hipEvent_t b)
   *ms = std::chrono::duration<float, std::milli>(b->t - a->t).count();
   return hipSuccess;
 }
-hipError_t hipGetDevice(int *d) { *d = 0; return hipSuccess; }
-hipError_t hipSetDevice(int) { return hipSuccess; }
+
+// two devices; a stream belongs to the one that was current when it was made
+struct emu_stream { int device; };
+static thread_local int emu_device = 0;
+static emu_pool emu_default_pools[2] = {{0, 0, 0}, {1, 0, 0}};
+static hipMemPool_t emu_pools[2] = {&emu_default_pools[0], &emu_default_pools[1]};
+hipMemPool_t emu_last_pool = nullptr;
+hipError_t hipGetDevice(int *d) { *d = emu_device; return hipSuccess; }
+hipError_t hipSetDevice(int d) { emu_device = d; return hipSuccess; }
+hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned)
+{
+  *s = new emu_stream{emu_device};
+  return hipSuccess;
+}
+hipError_t hipStreamDestroy(hipStream_t s) { delete s; return hipSuccess; }
+hipError_t hipStreamGetDevice(hipStream_t s, hipDevice_t *d)
+{
+  *d = s ? s->device : emu_device;
+  return hipSuccess;
+}
+hipError_t hipDeviceGetDefaultMemPool(hipMemPool_t *p, int d) { *p = &emu_default_pools[d]; return hipSuccess; }
+hipError_t hipDeviceGetMemPool(hipMemPool_t *p, int d) { *p = emu_pools[d]; return hipSuccess; }
+hipError_t hipDeviceSetMemPool(int d, hipMemPool_t p) { emu_pools[d] = p; return hipSuccess; }
+hipError_t hipMemPoolCreate(hipMemPool_t *p, const hipMemPoolProps *props)
+{
+  static std::vector<std::unique_ptr<emu_pool>> all;  // until the process ends
+  all.emplace_back(new emu_pool{props->location.id, 0, 0});
+  *p = all.back().get();
+  return hipSuccess;
+}
+hipError_t hipMemPoolDestroy(hipMemPool_t) { return hipSuccess; }
+hipError_t hipMemPoolSetAttribute(hipMemPool_t p, hipMemPoolAttr, void *v) { p->threshold = *(uint64_t *)v; return hipSuccess; }
+hipError_t hipMemPoolGetAttribute(hipMemPool_t p, hipMemPoolAttr, void *v) { *(uint64_t *)v = p->threshold; return hipSuccess; }
+hipError_t hipMemPoolTrimTo(hipMemPool_t, size_t) { return hipSuccess; }
+hipError_t hipMallocFromPoolAsync(void **p, size_t n, hipMemPool_t pool, hipStream_t)
+{
+  emu_last_pool = pool;
+  pool->allocations++;
+  return hipMalloc(p, n);
+}
+hipError_t hipMallocAsync(void **p, size_t n, hipStream_t s)
+{
+  int d;
+  hipStreamGetDevice(s, &d);
+  return hipMallocFromPoolAsync(p, n, emu_pools[d], s);
+}
 hipError_t hipDeviceGetAttribute(int *v, hipDeviceAttribute_t, int) { *v = 4; return hipSuccess; }

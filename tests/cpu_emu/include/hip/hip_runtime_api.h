@@ -23,6 +23,25 @@ typedef enum { hipMemcpyHostToHost, hipMemcpyHostToDevice, hipMemcpyDeviceToHost
 typedef enum { hipStreamCaptureStatusNone = 0, hipStreamCaptureStatusActive = 1 } hipStreamCaptureStatus;
 typedef enum { hipDeviceAttributeMultiprocessorCount = 0 } hipDeviceAttribute_t;
 typedef enum { hipFuncAttributeMaxDynamicSharedMemorySize = 0 } hipFuncAttribute;
+// memory pools: a pool remembers its device and its release threshold; memory
+// itself is the host's
+typedef int hipDevice_t;
+typedef struct emu_pool {
+  int device;
+  uint64_t threshold;
+  int allocations;
+} *hipMemPool_t;
+typedef enum { hipMemAllocationTypePinned = 1 } hipMemAllocationType;
+typedef enum { hipMemLocationTypeDevice = 1 } hipMemLocationType;
+typedef enum { hipMemPoolAttrReleaseThreshold = 4 } hipMemPoolAttr;
+typedef struct {
+  hipMemLocationType type;
+  int id;
+} hipMemLocation;
+typedef struct {
+  hipMemAllocationType allocType;
+  hipMemLocation location;
+} hipMemPoolProps;
 #define hipStreamNonBlocking 1
 #define hipEventDisableTiming 2
 #define hipHostMallocDefault 0
@@ -80,6 +99,18 @@ hipError_t hipEventSynchronize(hipEvent_t e);
 hipError_t hipEventElapsedTime(float *ms, hipEvent_t a, hipEvent_t b);
 hipError_t hipGetDevice(int *d);
 hipError_t hipSetDevice(int d);
+hipError_t hipStreamGetDevice(hipStream_t s, hipDevice_t *d);
+hipError_t hipDeviceGetDefaultMemPool(hipMemPool_t *p, int d);
+hipError_t hipDeviceGetMemPool(hipMemPool_t *p, int d);
+hipError_t hipDeviceSetMemPool(int d, hipMemPool_t p);
+hipError_t hipMemPoolCreate(hipMemPool_t *p, const hipMemPoolProps *props);
+hipError_t hipMemPoolDestroy(hipMemPool_t p);
+hipError_t hipMemPoolSetAttribute(hipMemPool_t p, hipMemPoolAttr a, void *v);
+hipError_t hipMemPoolGetAttribute(hipMemPool_t p, hipMemPoolAttr a, void *v);
+hipError_t hipMemPoolTrimTo(hipMemPool_t p, size_t keep);
+hipError_t hipMallocFromPoolAsync(void **p, size_t n, hipMemPool_t pool, hipStream_t s);
+// the pool of the latest stream-ordered allocation
+extern hipMemPool_t emu_last_pool;
 hipError_t hipDeviceGetAttribute(int *v, hipDeviceAttribute_t a, int dev);
 template <typename F>
 inline hipError_t hipFuncSetAttribute(F, hipFuncAttribute, int) { return hipSuccess; }
