@@ -769,10 +769,14 @@ int cukd_spatial_free(cukd_spatial_tree *tree, hipStream_t stream, const cukd_me
 // Spatial queries run in Morton order where the batch is large and the
 // points do not fit an L2: kNN-16 of 2M queries over 4M float4 8.5 -> 3.8 ms,
 // FCP of 1M over 300K 765 -> 505 us; the ordering of 150K queries costs FCP
-// over 300K more than it gives (186 -> 228 us).  Results are the same in any order.  A launch that is
-// being captured keeps the given order, since it must not allocate.
-static bool spatial_wants_order(const SpatialArgs &a, hipStream_t stream)
+// over 300K more than it gives (186 -> 228 us).  Results are the same in any
+// order.  The given order is kept where a query must not allocate: in a launch
+// that is being captured, and over a tree built with a caller's memory resource
+// (or of 8 dims, which has no room for the record: the order, two cells per
+// dim, gave 8 .. 12 % for 300K queries over 1M points there).
+static bool spatial_wants_order(const SpatialArgs &a, int may, hipStream_t stream)
 {
+  if (!(may & SPATIAL_MAY_ALLOCATE)) return false;
   const uint64_t bytes = (uint64_t)a.data.n * (uint64_t)a.data.stride;
   if (a.nq < (1 << 18) || bytes < SPATIAL_ORDER_MIN_BYTES) return false;
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
@@ -813,11 +817,12 @@ static int spatial_query(int traversal, int list_kind, int k, const cukd_spatial
   a.stats = g_stats;
   a.num_nodes = tree->num_nodes;
   // counted visits are the reference's
-  a.prune = !g_stats && spatial_prunable(tree, layout->num_dims);
+  const int may = spatial_may(tree, layout->num_dims);
+  a.prune = !g_stats && (may & SPATIAL_MAY_PRUNE);
   a.order = nullptr;
   void *otmp = nullptr;
   hipError_t e = hipSuccess;
-  if (spatial_wants_order(a, stream)) {
+  if (spatial_wants_order(a, may, stream)) {
     if (pool_malloc(&otmp, query_order_temp_bytes(nq), stream) == hipSuccess && otmp) {
       a.order = make_query_order(e, otmp, d_queries, nq, layout->num_dims, stream);
     } else {

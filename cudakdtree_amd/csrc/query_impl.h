@@ -501,7 +501,9 @@ struct SpatialArgs {
 // bytes of points from which large spatial batches run in Morton order: an
 // L2's size
 constexpr uint64_t SPATIAL_ORDER_MIN_BYTES = (uint64_t)4 << 20;
-bool spatial_prunable(const cukd_spatial_tree *tree, int D);
+// what the build recorded in the tree for its queries
+enum { SPATIAL_MAY_PRUNE = 1, SPATIAL_MAY_ALLOCATE = 2 };
+int spatial_may(const cukd_spatial_tree *tree, int D);
 hipError_t launch_spatial_query(int D, int method, const SpatialArgs &a, hipStream_t s);
 int spatial_build_impl(cukd_spatial_tree *tree, const void *d_points, int n, const cukd_layout &L,
                        int leaf_threshold, hipStream_t s, const MemResource &mem);

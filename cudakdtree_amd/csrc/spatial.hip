@@ -445,21 +445,27 @@ __global__ void k_sp_bounds_out(const SpNode *nodes, uint32_t *bounds, int D, bo
   }
 }
 
-// The bounds' last two words, unused below 8 dims, record that queries may
-// prune by box (k_spatial_query): no degenerate split, and no path of 50
-// inner nodes.  A tree without the record is queried without.
-enum : int32_t { SP_MARK = 0x70727562, SP_MARK2 = 0x786f622e };
-static void spatial_set_prunable(cukd_spatial_tree *tree, int D, bool ok)
+// The bounds' last two words, unused below 8 dims, record what queries may do
+// with the tree: prune by box (k_spatial_query), if it has no degenerate split
+// and no path of 50 inner nodes, and take scratch from the library's memory,
+// if the tree itself was built there and not with a caller's resource.  Without
+// the record they do neither.
+enum : int32_t { SP_MARK = 0x70727562, SP_MARK2 = 0x786f6200 };
+static void spatial_record(cukd_spatial_tree *tree, int D, bool prunable, const MemResource &mem)
 {
-  if (D >= CUKD_MAX_DIMS || !ok) return;
+  if (D >= CUKD_MAX_DIMS) return;
+  const bool scratch = !(mem.user && mem.user->malloc_fn);
   tree->ibounds[2 * CUKD_MAX_DIMS - 2] = SP_MARK;
-  tree->ibounds[2 * CUKD_MAX_DIMS - 1] = SP_MARK2;
+  tree->ibounds[2 * CUKD_MAX_DIMS - 1] =
+      SP_MARK2 | (prunable ? SPATIAL_MAY_PRUNE : 0) | (scratch ? SPATIAL_MAY_ALLOCATE : 0);
 }
 
-bool spatial_prunable(const cukd_spatial_tree *tree, int D)
+int spatial_may(const cukd_spatial_tree *tree, int D)
 {
-  return D < CUKD_MAX_DIMS && tree->ibounds[2 * CUKD_MAX_DIMS - 2] == SP_MARK &&
-         tree->ibounds[2 * CUKD_MAX_DIMS - 1] == SP_MARK2;
+  const int32_t w = tree->ibounds[2 * CUKD_MAX_DIMS - 1];
+  const int all = SPATIAL_MAY_PRUNE | SPATIAL_MAY_ALLOCATE;
+  if (D >= CUKD_MAX_DIMS || tree->ibounds[2 * CUKD_MAX_DIMS - 2] != SP_MARK) return 0;
+  return (w & ~all) == SP_MARK2 ? w & all : 0;
 }
 
 enum { SP_DEPTH = 50 };  // the reference's traversal stack (fcp.h:265)
@@ -595,7 +601,7 @@ static int spatial_build_rounds(cukd_spatial_tree *tree, const void *d_points, i
       if (e == hipSuccess) e = hipStreamSynchronize(s);
       if (e == hipSuccess) {
         for (int i = 0; i < 2 * CUKD_MAX_DIMS; i++) tree->ibounds[i] = i < 2 * D ? (int32_t)hb[i] : 0;
-        spatial_set_prunable(tree, D, levels <= SP_DEPTH && hb[2 * D] == 0u);
+        spatial_record(tree, D, levels <= SP_DEPTH && hb[2 * D] == 0u, mem);
         tree->nodes = out_nodes;
         tree->prim_ids = out_prims;
         tree->data = d_points;

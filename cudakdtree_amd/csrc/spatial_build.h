@@ -925,7 +925,7 @@ static int spatial_build_items(cukd_spatial_tree *tree, const uint8_t *pts, int 
     tree->ibounds[i] = i < 2 * D ? (int32_t)hw[SPB_LEVELS + i] : 0;
   int levels = 0;
   while (levels < SPB_LEVELS && hw[levels]) levels++;
-  spatial_set_prunable(tree, D, levels <= SP_DEPTH && h.degen == 0u);
+  spatial_record(tree, D, levels <= SP_DEPTH && h.degen == 0u, mem);
   tree->nodes = out_nodes;
   tree->prim_ids = out_prims;
   tree->data = pts;

@@ -268,7 +268,9 @@ int cukd_spatial_free(cukd_spatial_tree *tree, hipStream_t stream,
                       const cukd_mem_resource *mem);
 
 /* Spatial FCP / kNN (fcp.h:256-427, knn.h:566-752); traversal is
- * CUKD_STACK_BASED or CUKD_CCT.  Ids are original point indices. */
+ * CUKD_STACK_BASED or CUKD_CCT.  Ids are original point indices.  Large
+ * batches over a tree built without a memory resource run in Morton order,
+ * with scratch of the library's; over any other tree nothing is allocated. */
 int cukd_spatial_fcp(int traversal, const cukd_spatial_tree *tree,
                      const cukd_layout *layout, const float *d_queries,
                      int32_t nq, float cutoff, int32_t *d_ids, float *d_dist2,

@@ -310,6 +310,34 @@ bool pool_case(const char *what)
   return ok;
 }
 
+int own_malloc(void *, void **p, size_t n, hipStream_t) { return hipMalloc(p, n); }
+int own_free(void *, void *p, hipStream_t) { return hipFree(p); }
+
+// A large batch over a spatial tree built with the caller's memory resource
+// allocates nothing; over one built without, it is Morton-ordered.
+bool spatial_scratch_case(bool own)
+{
+  const int n = 16400, nq = 1 << 18;
+  const cukd_layout L{3, CUKD_SCALAR_F32, 256, 0, -1, 4};
+  const cukd_mem_resource res{nullptr, own_malloc, own_free};
+  uint64_t seed = 33;
+  std::vector<float> pts((size_t)n * 64, 0.f), q;
+  for (int i = 0; i < n; i++)
+    for (int d = 0; d < 3; d++) pts[(size_t)i * 64 + d] = unit(seed);
+  for (int i = 0; i < 3 * nq; i++) q.push_back(unit(seed));
+  Dev<float> dp(pts), dq(q);
+  Dev<int32_t> di((size_t)nq);
+  cukd_spatial_tree t;
+  if (cukd_spatial_build(&t, dp.p, n, &L, 0, nullptr, own ? &res : nullptr) != CUKD_OK) return false;
+  const size_t from = emu_launches.size();
+  emu_last_pool = nullptr;
+  bool ok = cukd_spatial_fcp(CUKD_STACK_BASED, &t, &L, dq.p, nq, 0.001f, di.p, nullptr,
+                             nullptr) == CUKD_OK &&
+            (emu_last_pool == nullptr) == own && (launches_of("k_qplace", from) == 0) == own;
+  cukd_spatial_free(&t, nullptr, own ? &res : nullptr);
+  return ok;
+}
+
 }  // namespace
 
 int main(int argc, char **argv)
@@ -345,6 +373,9 @@ int main(int argc, char **argv)
   for (const char *what : {"nothing chosen", "stream of another device", "a current pool",
                            "a default pool that keeps", "nothing chosen"})
     cases.push_back({std::string("memory pool, ") + what, [=] { return pool_case(what); }});
+  for (bool own : {false, true})
+    cases.push_back({std::string("scratch of spatial queries, ") + (own ? "caller's" : "library's") + " memory",
+                     [=] { return spatial_scratch_case(own); }});
   int fail = 0;
   for (auto &c : cases)
     if (only.empty() || c.name.find(only) != std::string::npos) {
