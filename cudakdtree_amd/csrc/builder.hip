@@ -2000,12 +2000,14 @@ __global__ __launch_bounds__(NT) void k_finish_rank(
 // The launches above spread one subtree over many workgroups, so they meet
 // through memory at five kernel boundaries a level (about 45 us for a level
 // of 100K points, whatever its size).  A subtree of at most WG_MAX elements
-// is taken by one workgroup instead, with its keys in registers:
+// is taken by one workgroup instead, with the word being resolved in LDS:
 //  * the range that holds the pivot's key shrinks by 2048 linear bins at a
 //    time until at most WG_CAND elements lie in it (one pass, nearly always;
 //    where more elements share one key, their next word takes over);
 //  * those few are ranked against each other by their whole keys, one lane
-//    each, which finds the pivot and settles ties;
+//    each, which finds the pivot and the sides of the elements around it; tied
+//    ones bring their other words into LDS first (read from memory for each
+//    pair, a level of a 64-step grid took 80 us more);
 //  * the partition ranks by ballots in (item, wave, lane) order, as
 //    k_partition does.
 // The tree is the same: a level depends on the pivots only, not on the order
@@ -2013,10 +2015,10 @@ __global__ __launch_bounds__(NT) void k_finish_rank(
 // Bound by barriers and memory latency: 13 us for a level of 800-element
 // subtrees, 20 at 3K, 30 at 6K and 47 at 12.5K, where the five launches take
 // 42 .. 49 us; a level of 1024 subtrees of 9.8K (10M points) takes 100 us less.
-// Builds: 2000 points 159 -> 118 us, 10K 286 -> 193, 100K 462 -> 377.
+// Builds: 2000 points 159 -> 118 us, 10K 286 -> 193, 100K 462 -> 377; 40K
+// points of a 64-step grid 836 -> 674, of an 8-step one 880 -> 881.
 enum { WG_NT = 1024, WG_E = 16, WG_MAX = WG_NT * WG_E, WG_BINS = 2048, WG_CAND = 256 };
 
-//
 // SW: elements of at most SW words pass through registers (0: any size).
 template <bool EXPLICIT, int SW>
 __global__ __launch_bounds__(WG_NT) void k_level_wg(TreeSet<LvlTree> set, int level,
@@ -2030,10 +2032,11 @@ __global__ __launch_bounds__(WG_NT) void k_level_wg(TreeSet<LvlTree> set, int le
   __shared__ uint32_t s_wsum[NW], s_lo[NW], s_hi[NW];
   __shared__ uint32_t s_pick[3];  // bin, elements of the lower bins, elements of the bin
   __shared__ uint32_t s_cval[WG_CAND], s_cpos[WG_CAND], s_ncand;
-  __shared__ uint32_t s_pw[MAX_WORDS];  // the pivot's words
-  __shared__ int s_pivot;               // its position
+  __shared__ int s_pivot;               // the pivot's position
   __shared__ uint32_t s_cnt[2 * WG_E * NW];
-  __shared__ uint8_t s_rank[WG_MAX];    // rank of an element among its wave's of one item and side
+  // a candidate's side (1: left), then the rank of an element among its wave's
+  // of one item and side
+  __shared__ uint8_t s_rank[WG_MAX];
   __shared__ uint32_t s_cdim[2];
   __shared__ SegState s_st;
   __shared__ LvlTree s_tree;
@@ -2087,6 +2090,7 @@ __global__ __launch_bounds__(WG_NT) void k_level_wg(TreeSet<LvlTree> set, int le
   // the candidates: elements of 'mask' whose word w lies in [lo, hi]
   uint32_t rem = (uint32_t)subtree_size(2 * node + 1, tr.n);  // the pivot's rank among them
   uint32_t cnt = (uint32_t)m, lo = 0u, hi = 0u;
+  uint32_t below = 0;  // elements out of 'mask' that are left of the pivot
   int w = 0;
   for (;;) {
     lo = 0xffffffffu;
@@ -2147,12 +2151,18 @@ __global__ __launch_bounds__(WG_NT) void k_level_wg(TreeSet<LvlTree> set, int le
     for (int e = 0; e < WG_E; e++) {
       const int p = e * WG_NT + tid;
       if (!((mask >> e) & 1u)) continue;
-      if (s_v[p] != lo) mask &= ~(1u << e);
-      else s_v[p] = word(w, p);
+      const uint32_t x = s_v[p];
+      if (x == lo) {
+        s_v[p] = word(w, p);
+      } else {
+        mask &= ~(1u << e);
+        below |= x < lo ? 1u << e : 0u;
+      }
     }
     __syncthreads();
   }
-  // rank the candidates among themselves by their remaining words
+  // rank the candidates among themselves; those of equal words by their next
+  // ones, which they bring into LDS (a list of lists of words, in s_hist)
 #pragma unroll 4
   for (int e = 0; e < WG_E; e++) {
     if (!((mask >> e) & 1u)) continue;
@@ -2163,34 +2173,38 @@ __global__ __launch_bounds__(WG_NT) void k_level_wg(TreeSet<LvlTree> set, int le
     s_cpos[i] = (uint32_t)(e * WG_NT + tid);
   }
   __syncthreads();
+  static_assert(CUKD_MAX_DIMS * WG_CAND <= WG_BINS, "the candidates' words fit s_hist");
+  uint32_t crank = 0, cval = 0;
+  bool tied = false;
   if ((uint32_t)tid < cnt) {
-    const uint32_t mine = s_cval[tid];
-    const int p = (int)s_cpos[tid];
-    uint32_t r = 0;
+    cval = s_cval[tid];
     for (uint32_t j = 0; j < cnt; j++) {
       const uint32_t o = s_cval[j];
-      bool less = o < mine;
-      if (o == mine && (int)j != tid) {
-        const int q = (int)s_cpos[j];
-        for (int x = w + 1; x <= clen; x++) {
-          const uint32_t a = word(x, q), b = word(x, p);
-          if (a != b) {
-            less = a < b;
-            break;
-          }
-        }
-      }
-      r += less ? 1u : 0u;
+      crank += o < cval ? 1u : 0u;
+      tied = tied || (o == cval && (int)j != tid);
     }
-    if (r == rem) s_pivot = p;
+    if (tied)
+      for (int x = w + 1; x <= clen; x++)
+        s_hist[(x - 1) * WG_CAND + tid] = word(x, (int)s_cpos[tid]);
+  }
+  __syncthreads();
+  if ((uint32_t)tid < cnt) {
+    for (uint32_t j = 0; tied && j < cnt; j++) {
+      if (s_cval[j] != cval) continue;
+      for (int x = w; x < clen; x++) {
+        const uint32_t a = s_hist[x * WG_CAND + j], b = s_hist[x * WG_CAND + tid];
+        if (a == b) continue;
+        crank += a < b ? 1u : 0u;
+        break;
+      }
+    }
+    if (crank == rem) s_pivot = (int)s_cpos[tid];
+    s_rank[s_cpos[tid]] = crank < rem ? 1 : 0;
   }
   __syncthreads();
   const int piv = s_pivot;
-  if (tid <= clen) s_pw[tid] = tid == 0 ? key[piv] : word(tid, piv);
-  __syncthreads();
-  const uint32_t pk = s_pw[0];
   if (EXPLICIT && tid == 0) {
-    s_st.fixed[0] = pk;
+    s_st.fixed[0] = key[piv];
     write_child_domains(s_st, st + tr.cseg, s, L, isf);
     s_cdim[0] = st[tr.cseg + 2 * s].dim;
     s_cdim[1] = st[tr.cseg + 2 * s + 1].dim;
@@ -2208,16 +2222,8 @@ __global__ __launch_bounds__(WG_NT) void k_level_wg(TreeSet<LvlTree> set, int le
     const int p = e * WG_NT + tid;
     bool l = false, r = false;
     if (p < m && p != piv) {
-      const uint32_t ke = w == 0 ? s_v[p] : key[p];
-      l = ke < pk;
-      if (ke == pk)
-        for (int x = 1; x <= clen; x++) {
-          const uint32_t a = word(x, p);
-          if (a != s_pw[x]) {
-            l = a < s_pw[x];
-            break;
-          }
-        }
+      const uint32_t x = s_v[p];
+      l = (mask >> e) & 1u ? x < lo || (x <= hi && s_rank[p]) : (below >> e) & 1u;
       r = !l;
     }
     const uint64_t ml = __ballot(l), mr = __ballot(r);
