@@ -2017,7 +2017,14 @@ __global__ __launch_bounds__(NT) void k_finish_rank(
 // 42 .. 49 us; a level of 1024 subtrees of 9.8K (10M points) takes 100 us less.
 // Builds: 2000 points 159 -> 118 us, 10K 286 -> 193, 100K 462 -> 377; 40K
 // points of a 64-step grid 836 -> 674, of an 8-step one 880 -> 881.
-enum { WG_NT = 1024, WG_E = 16, WG_MAX = WG_NT * WG_E, WG_BINS = 2048, WG_CAND = 256 };
+//
+// Elements of more than WG_REG_WORDS words take this kernel while the subtree
+// has at most WG_BYTES: one workgroup moves 30 .. 40 GB/s, so a level of large
+// subtrees is faster spread over the chip.  16K points: 32 bytes each 301 -> 240
+// us, 48 bytes 350 -> 284, 96 bytes (1.5 MB) 429 -> 466, 256 bytes 718 -> 1041;
+// 3000 points (768 KB) of 256 bytes 491 -> 481.
+enum { WG_NT = 1024, WG_E = 16, WG_MAX = WG_NT * WG_E, WG_BINS = 2048, WG_CAND = 256,
+       WG_REG_WORDS = 5, WG_BYTES = 768 << 10 };
 
 // SW: elements of at most SW words pass through registers (0: any size).
 template <bool EXPLICIT, int SW>
@@ -2250,48 +2257,84 @@ __global__ __launch_bounds__(WG_NT) void k_level_wg(TreeSet<LvlTree> set, int le
   const int W = L.stride >> 2, cw0 = L.point_offset >> 2;
   const int base0 = gn.offset(2 * s), base1 = gn.offset(2 * s + 1);
   const uint32_t cd0 = s_cdim[0], cd1 = s_cdim[1];
-  // WG_BATCH elements at a time, all their loads in flight before a store
-  enum { WG_BATCH = 4 };
-  for (int e0 = 0; e0 < WG_E; e0 += WG_BATCH) {
-    if (e0 * WG_NT >= m) break;
-    uint32_t x[WG_BATCH][SW > 0 ? SW : 1], id[WG_BATCH];
-    int dst[WG_BATCH];
-    bool left[WG_BATCH];
+  auto target = [&](int e, bool left) {
+    return (left ? base0 : base1) + (int)s_cnt[(left ? 0 : WG_E * NW) + e * NW + wave] +
+           (int)s_rank[e * WG_NT + tid];
+  };
+  if constexpr (SW > 0) {
+    // WG_BATCH elements at a time, all their loads in flight before a store
+    enum { WG_BATCH = 4 };
+    for (int e0 = 0; e0 < WG_E; e0 += WG_BATCH) {
+      if (e0 * WG_NT >= m) break;
+      uint32_t x[WG_BATCH][SW], id[WG_BATCH];
+      int dst[WG_BATCH];
+      bool left[WG_BATCH];
 #pragma unroll
-    for (int i = 0; i < WG_BATCH; i++) {
-      const int e = e0 + i, p = e * WG_NT + tid;
-      left[i] = (lefts >> e) & 1u;
-      const bool mv = left[i] || ((rights >> e) & 1u);
-      dst[i] = -1;
-      id[i] = 0;
-      if (mv) {
-        id[i] = idx[p];
-        dst[i] = (left[i] ? base0 : base1) +
-                 (int)s_cnt[(left[i] ? 0 : WG_E * NW) + e * NW + wave] + s_rank[e * WG_NT + tid];
+      for (int i = 0; i < WG_BATCH; i++) {
+        const int e = e0 + i, p = e * WG_NT + tid;
+        left[i] = (lefts >> e) & 1u;
+        const bool mv = left[i] || ((rights >> e) & 1u);
+        dst[i] = mv ? target(e, left[i]) : -1;
+        id[i] = mv ? idx[p] : 0u;
+#pragma unroll
+        for (int j = 0; j < SW; j++)
+          x[i][j] = mv && j < W ? ((const uint32_t *)(data + (size_t)p * L.stride))[j] : 0u;
       }
 #pragma unroll
-      for (int j = 0; j < SW; j++)
-        x[i][j] = mv && j < W ? ((const uint32_t *)(data + (size_t)p * L.stride))[j] : 0u;
-    }
-#pragma unroll
-    for (int i = 0; i < WG_BATCH; i++) {
-      if (dst[i] < 0) continue;
-      uint32_t *to = (uint32_t *)(ndata + (size_t)dst[i] * L.stride);
-      const int kw = cw0 + (int)(left[i] ? cd0 : cd1);
-      uint32_t kv = 0;
-      if (SW > 0) {
+      for (int i = 0; i < WG_BATCH; i++) {
+        if (dst[i] < 0) continue;
+        uint32_t *to = (uint32_t *)(ndata + (size_t)dst[i] * L.stride);
+        const int kw = cw0 + (int)(left[i] ? cd0 : cd1);
+        uint32_t kv = 0;
 #pragma unroll
         for (int j = 0; j < SW; j++) {
           if (j < W) to[j] = x[i][j];
           kv = j == kw ? x[i][j] : kv;
         }
-      } else {
-        const uint32_t *src = (const uint32_t *)(data + (size_t)((e0 + i) * WG_NT + tid) * L.stride);
-        for (int j = 0; j < W; j++) to[j] = src[j];
-        kv = src[kw];
+        nidx[dst[i]] = id[i];
+        if (tr.more) nkey[dst[i]] = ordered_key(kv, isf);
       }
-      nidx[dst[i]] = id[i];
-      if (tr.more) nkey[dst[i]] = ordered_key(kv, isf);
+    }
+  } else {
+    // Consecutive threads take consecutive words, so that loads and stores run
+    // along the elements; an element's place waits in LDS, with its side in the
+    // top bit (a lane per element: 40K points of 96 bytes 549 -> 1239 us).
+    enum { WG_BATCH = 8 };
+    const uint32_t NONE = 0xffffffffu;
+    for (int e = 0; e * WG_NT < m && e < WG_E; e++) {
+      const int p = e * WG_NT + tid;
+      if (p >= m) continue;
+      const bool left = (lefts >> e) & 1u;
+      s_v[p] = NONE;
+      if (p == piv) continue;
+      const int dst = target(e, left);
+      s_v[p] = (uint32_t)dst | (left ? 0u : 0x80000000u);
+      nidx[dst] = idx[p];
+    }
+    __syncthreads();
+    const uint32_t *src = (const uint32_t *)data;
+    uint32_t *to = (uint32_t *)ndata;
+    const int words = m * W, dp = WG_NT / W, dj = WG_NT % W;
+    int p = tid / W, j = tid % W;
+    for (int i = tid; i < words; i += WG_NT * WG_BATCH) {
+      uint32_t x[WG_BATCH];
+#pragma unroll
+      for (int b = 0; b < WG_BATCH; b++) x[b] = i + b * WG_NT < words ? src[i + b * WG_NT] : 0u;
+#pragma unroll
+      for (int b = 0; b < WG_BATCH; b++) {
+        const uint32_t t = i + b * WG_NT < words ? s_v[p] : NONE;
+        if (t != NONE) {
+          const int dst = (int)(t & 0x7fffffffu);
+          to[(size_t)dst * W + j] = x[b];
+          if (tr.more && j == cw0 + (int)(t >> 31 ? cd1 : cd0)) nkey[dst] = ordered_key(x[b], isf);
+        }
+        p += dp;
+        j += dj;
+        if (j >= W) {
+          j -= W;
+          p++;
+        }
+      }
     }
   }
   if (tid < W)
@@ -2468,7 +2511,8 @@ int make_forest_plan(ForestPlan &P, const long long *off, int ntrees, const cukd
     for (const LvlTree &x : v) {
       LevelGeom g;
       g.init(x.n, l);
-      wg = wg && g.size(0) <= WG_MAX;
+      wg = wg && g.size(0) <= WG_MAX &&
+           (L.stride <= 4 * WG_REG_WORDS || (long long)g.size(0) * L.stride <= WG_BYTES);
     }
     P.lvl_wg.push_back(wg ? 1 : 0);
     P.lvl.push_back(v);
@@ -2656,9 +2700,10 @@ int forest_build_run(const ForestPlan &P, void *d_points, void *d_bounds, uint8_
         make_set(P, ws, P.tables ? P.off_tab_lvl[level] : 0, P.lvl[level]);
     if (level >= wg0) {
       const int W = L.stride >> 2;
-      auto kw = expl ? (W <= 5 ? k_level_wg<true, 5> : k_level_wg<true, 0>)
+      auto kw = expl ? (W <= WG_REG_WORDS ? k_level_wg<true, WG_REG_WORDS> : k_level_wg<true, 0>)
                      : (W <= 3 ? k_level_wg<false, 3>
-                               : (W <= 5 ? k_level_wg<false, 5> : k_level_wg<false, 0>));
+                               : (W <= WG_REG_WORDS ? k_level_wg<false, WG_REG_WORDS>
+                                                    : k_level_wg<false, 0>));
       hipLaunchKernelGGL(kw, dim3(P.lvl_segs[level]), dim3(WG_NT), 0, s, set, level,
                          (const uint32_t *)kcur, (const uint8_t *)dcur, (const uint32_t *)icur, st,
                          dnext, inext, knext, pts, L);
