@@ -485,7 +485,7 @@ int spatial_build_impl(cukd_spatial_tree *tree, const void *d_points, int n, con
 {
   const uint32_t thr = leaf_threshold <= 0 ? 8u : (uint32_t)leaf_threshold;
   (void)hipGetLastError();  // an earlier call's error is no launch's below
-  if (n > 0) {
+  if (n > 0 && (uint32_t)n > thr) {  // one leaf takes fewer launches round by round
     const uint8_t *pts = (const uint8_t *)d_points;
     bool deep = false;
     int rc;
@@ -504,8 +504,8 @@ int spatial_build_impl(cukd_spatial_tree *tree, const void *d_points, int n, con
   return spatial_build_rounds(tree, d_points, n, L, thr, s, mem);
 }
 
-// Round by round over all open nodes: trees of more than SPB_LEVELS levels,
-// and the empty one.
+// Round by round over all open nodes: trees of more than SPB_LEVELS levels, and
+// those of one leaf (5 points 200 us, 228 the other way).
 static int spatial_build_rounds(cukd_spatial_tree *tree, const void *d_points, int n,
                                 const cukd_layout &L, uint32_t thr, hipStream_t s,
                                 const MemResource &mem)

@@ -813,10 +813,10 @@ static int spatial_build_items(cukd_spatial_tree *tree, const uint8_t *pts, int 
   const uint32_t small = thr > (uint32_t)SPB_T ? thr : (uint32_t)SPB_T;
   const bool isf = L.scalar_type == CUKD_SCALAR_F32;
   const int gn = (n + 255) / 256;
-  // more dynamic LDS than a kernel may take unasked
-  hipError_t e = hipFuncSetAttribute((const void *)k_spb_small<D>,
-                                     hipFuncAttributeMaxDynamicSharedMemorySize,
-                                     (int)spb_lds(D, thr));
+  hipError_t e = hipSuccess;
+  if (spb_lds(D, thr) > 65536)  // more than a kernel may take unasked
+    e = hipFuncSetAttribute((const void *)k_spb_small<D>,
+                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)spb_lds(D, thr));
 
   CUKD_LAUNCH(e, k_spb_init, dim3(gn), dim3(256), 0, s, nodes, boxes, st, pp0, pn0,
               n, D);
