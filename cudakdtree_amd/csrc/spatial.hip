@@ -829,10 +829,16 @@ __global__ __launch_bounds__(256) void k_spatial_query(const cukd_spatial_node *
 
 // The traversals of cukd/spatial-kdtree.h as they stand, with lists whose
 // keys are compared as integers: for NaN cutoffs, whose keys have no order
-// as doubles, for trees of 2^29 nodes and more, and for the closest point of
-// many queries in a small tree, where reading single points wins (1M queries
-// over 100K float4: 338 us here, 395 us above).  The first 16 entries of the
-// stack-based FCP's stack are LDS columns.
+// as doubles, for trees of 2^29 nodes and more, and where reading single points
+// wins:
+//  * one dim, few entries, below 2^18 queries, over 1K .. 1M points: FCP takes
+//    0.72 .. 1.02 times the kernel above, k = 1 and 2 0.74 .. 1.1, k = 4 0.71 ..
+//    1.2 with the list in registers; k = 3, and 5 and more, 1.0 .. 2.2 times;
+//  * the closest point of 2^19 queries and more in a small tree, if half of
+//    them find none: 1M queries over 100K float4 330 us here, 386 above.  Where
+//    most find one it is 563 against 359 (2^19 queries), but never slower than
+//    it has been.
+// The first 16 entries of the stack-based FCP's stack are LDS columns.
 template <bool CCT, class R> struct SpStackCols {
   enum { value = (CCT || ResultOps<R>::kLds) ? 0 : 16 };
 };
@@ -893,7 +899,9 @@ static hipError_t launch_spatial_m(const SpatialArgs &a, hipStream_t s)
 {
   const bool small_fcp = !CCT && a.list_kind < 0 && a.nq >= (1 << 19) &&
                          (uint64_t)a.data.n * (uint64_t)a.data.stride < SPATIAL_ORDER_MIN_BYTES;
-  if (a.cutoff != a.cutoff || a.num_nodes > (1 << SP_DIM_SHIFT) || small_fcp) {
+  const bool line = D == 1 && a.nq < (1 << 18) &&
+                    (a.k <= 2 || (a.k == 4 && a.list_kind == CUKD_LIST_FIXED));
+  if (a.cutoff != a.cutoff || a.num_nodes > (1 << SP_DIM_SHIFT) || small_fcp || line) {
     const int nt = 128, blocks = (a.nq + nt - 1) / nt;
     // dynamic LDS: k 64-bit words per lane (64 KiB at k = 64), or the stack
     // columns (16 KiB)
@@ -906,6 +914,7 @@ static hipError_t launch_spatial_m(const SpatialArgs &a, hipStream_t s)
                      a.stats)
     if (a.list_kind < 0) CUKD_SPQ(cukd::FCPResult);
     else if (a.list_kind == CUKD_LIST_HEAP) CUKD_SPQ(LdsHeapList);
+    else if (D == 1 && a.k == 4) CUKD_SPQ(cukd::FixedCandidateList<D == 1 ? 4 : 1>);
     else CUKD_SPQ(DynFixedList);
 #undef CUKD_SPQ
     return hipGetLastError();
