@@ -2684,7 +2684,8 @@ int forest_build_run(const ForestPlan &P, void *d_points, void *d_bounds, uint8_
   // levels from 'wg0' on run one workgroup per subtree
   int wg0 = P.max_L0;
   while (wg0 > 0 && P.lvl_wg[wg0 - 1]) wg0--;
-  hipLaunchKernelGGL(k_copy_in, dim3(P.in_tiles), dim3(COPY_NT), 0, s, in, dataA, idxA,
+  const int copy_nt = P.max_n > COPY_NT / 4 ? COPY_NT : COPY_NT / 4;
+  hipLaunchKernelGGL(k_copy_in, dim3(P.in_tiles), dim3(copy_nt), 0, s, in, dataA, idxA,
                      P.max_L0 > 0 ? keyA : (uint32_t *)nullptr, (const uint8_t *)pts, L,
                      (const SegState *)st, expl ? 1 : 0, h0,
                      wg0 > 0 ? (P.zero_end - P.off_hist) / 4 : 0);
