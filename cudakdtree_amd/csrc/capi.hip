@@ -387,7 +387,10 @@ static int run_queries(QueryArgs a, int D, int traversal, int flags, const MemRe
                        void *order_ws, size_t order_ws_bytes, bool repeatable,
                        hipStream_t stream, const char *what)
 {
-  TuneVal cfg{0, (flags & CUKD_QUERY_SORT) ? 1 : 0};
+  // one wave's queries need no order among them (kNN-2 of 1 query, ordered: 36 us
+  // at one time, 40 with the present ordering kernels, 12 without)
+  const bool orderable = a.nq > 64;
+  TuneVal cfg{0, orderable && (flags & CUKD_QUERY_SORT) ? 1 : 0};
   a.box = !(flags & CUKD_QUERY_ONE_PER_LANE);
   bool tune = false;
   TuneKey key;
@@ -396,7 +399,7 @@ static int run_queries(QueryArgs a, int D, int traversal, int flags, const MemRe
   key.trav = traversal;
   key.list = a.list_kind;
   key.k = a.k;
-  key.bucket = log2_bucket(a.nq);
+  key.bucket = log2_bucket(a.nq - 1);  // up to 64, no bucket has orderable batches
   key.forest = a.fq.seg_off != nullptr;
   key.box = box_ok(a);
   if (flags & CUKD_QUERY_AUTOTUNE) {
@@ -407,7 +410,7 @@ static int run_queries(QueryArgs a, int D, int traversal, int flags, const MemRe
   }
   void *otmp = nullptr;
   bool owned = false;
-  if (cfg.sort || tune) {
+  if (cfg.sort || (tune && orderable)) {
     const size_t need = query_order_temp_bytes(a.nq);
     if (order_ws && order_ws_bytes >= need) {
       otmp = order_ws;
@@ -424,7 +427,7 @@ static int run_queries(QueryArgs a, int D, int traversal, int flags, const MemRe
     float best = 3.4e38f;
     TuneVal bestv = cfg;
     const int blocks[3] = {64, 128, 256};
-    for (int sort = 0; sort < 2 && e == hipSuccess; sort++)
+    for (int sort = 0; sort <= (orderable ? 1 : 0) && e == hipSuccess; sort++)
       for (int bi = 0; bi < 3 && e == hipSuccess; bi++) {
         QueryArgs v = a;
         v.block = blocks[bi];

@@ -310,6 +310,30 @@ bool pool_case(const char *what)
   return ok;
 }
 
+// A batch of one wave is never ordered and allocates nothing; larger ones are.
+bool small_batch_case(int nq, int flags)
+{
+  const int n = 400, k = 2 + flags;  // its own tuned choice
+  const cukd_layout L = floats(3);
+  const oc_layout O = ocl(L);
+  uint64_t seed = 17;
+  std::vector<float> pts, q;
+  for (int i = 0; i < 3 * n; i++) pts.push_back(unit(seed));
+  for (int i = 0; i < 3 * nq; i++) q.push_back(unit(seed));
+  oc_build_host(pts.data(), n, &O, nullptr);
+  Dev<float> dt(pts), dq(q), dd((size_t)nq * k);
+  Dev<int32_t> di((size_t)nq * k);
+  std::vector<int32_t> ri((size_t)nq * k);
+  std::vector<float> rd((size_t)nq * k);
+  oc_knn(OC_STACK_BASED, OC_LIST_FIXED, k, pts.data(), n, &O, nullptr, q.data(), nq, INFINITY,
+         ri.data(), rd.data(), nullptr, nullptr, 1);
+  emu_last_pool = nullptr;
+  return cukd_knn(CUKD_STACK_BASED, CUKD_LIST_FIXED, k, dt.p, n, &L, nullptr, dq.p, nq, INFINITY,
+                  di.p, dd.p, nullptr, flags, nullptr, nullptr) == CUKD_OK &&
+         di.same(ri) && dd.same(rd) && (launches_of("k_qplace", 0) > 0) == (nq > 64) &&
+         (emu_last_pool != nullptr) == (nq > 64);
+}
+
 int own_malloc(void *, void **p, size_t n, hipStream_t) { return hipMalloc(p, n); }
 int own_free(void *, void *p, hipStream_t) { return hipFree(p); }
 
@@ -373,6 +397,10 @@ int main(int argc, char **argv)
   for (const char *what : {"nothing chosen", "stream of another device", "a current pool",
                            "a default pool that keeps", "nothing chosen"})
     cases.push_back({std::string("memory pool, ") + what, [=] { return pool_case(what); }});
+  for (int nq : {1, 63, 64, 65})
+    for (int flags : {CUKD_QUERY_SORT, CUKD_QUERY_AUTOTUNE, CUKD_QUERY_SORT | CUKD_QUERY_AUTOTUNE})
+      cases.push_back({"order of small batches, nq=" + std::to_string(nq) + " flags=" + std::to_string(flags),
+                       [=] { return small_batch_case(nq, flags); }});
   for (bool own : {false, true})
     cases.push_back({std::string("scratch of spatial queries, ") + (own ? "caller's" : "library's") + " memory",
                      [=] { return spatial_scratch_case(own); }});

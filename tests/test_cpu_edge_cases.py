@@ -16,7 +16,8 @@ def edge_test():
     return os.path.join(EMU, "_build", "edge_test")
 
 
-@pytest.mark.parametrize("cases", ["spatial centre", "spatial overflow", "autotune", "refused launch", "memory pool", "scratch"])
+@pytest.mark.parametrize("cases", ["spatial centre", "spatial overflow", "autotune", "refused launch", "memory pool", "scratch",
+                                   "order of small"])
 def test_edge_cases(edge_test, cases):
     r = subprocess.run([edge_test, cases], capture_output=True, text=True, timeout=600)
     assert r.returncode == 0 and " ok\n" in r.stdout and "ALL OK" in r.stdout, \
