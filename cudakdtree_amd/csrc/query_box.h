@@ -13,8 +13,8 @@
 //  subtree has a computed dist2 of at least that sum: above the cull, where
 //  no list accepts it.  Skipping it changes no accepted candidate, no later
 //  cull and no order.  (An equal distance is not skipped: a smaller id could
-//  still be accepted.)  CPU count over 10M uniform points: 95 visits per
-//  query instead of 112 for kNN-8, 273 instead of 357 for k = 50, and a
+//  still be accepted.)  CPU count over 10M uniform points: 96 visits per
+//  query instead of 112 for kNN-8, 276 instead of 357 for k = 50, and a
 //  fifth of them for queries far from clustered points.
 //
 //  Planes in LDS.  Row r of a lane's LDS column holds diff*diff of the far
@@ -24,7 +24,7 @@
 //  the far children on the path (mask 'far'), the deepest one per dim.
 //
 // What bounds it: vector issue at partial lane use (a wave runs 170
-// iterations for 95 visits per lane at kNN-8) and one line access per lane
+// iterations for 96 visits per lane at kNN-8) and one line access per lane
 // and visit; a small batch is one chain of iterations of 0.3 .. 0.5 us.
 // Measured on 1M Morton-ordered queries over 10M uniform float3, kernel time
 // before (two queries per lane, planes only; k = 20 and up: lists in LDS,
