@@ -46,7 +46,11 @@ static hipMemPool_t library_pool(hipStream_t s)
   hipDevice_t dev = 0;
   hipMemPool_t def = nullptr, current = nullptr, pool = nullptr;
   uint64_t keep = 0;
-  if (hipStreamIsCapturing(s, &st) != hipSuccess || hipStreamGetDevice(s, &dev) != hipSuccess ||
+  // the stock streams are the current device's, and the runtime ends in a
+  // segmentation fault when asked for the device of hipStreamLegacy
+  const bool stock = s == nullptr || s == hipStreamLegacy || s == hipStreamPerThread;
+  if (hipStreamIsCapturing(s, &st) != hipSuccess ||
+      (stock ? hipGetDevice(&dev) : hipStreamGetDevice(s, &dev)) != hipSuccess ||
       hipDeviceGetDefaultMemPool(&def, dev) != hipSuccess ||
       hipDeviceGetMemPool(&current, dev) != hipSuccess ||
       hipMemPoolGetAttribute(def, hipMemPoolAttrReleaseThreshold, &keep) != hipSuccess) {

@@ -288,9 +288,13 @@ bool pool_case(const char *what)
   const bool other = !strcmp(what, "stream of another device");
   const int dev = other ? 1 : 0;
   hipSetDevice(dev);
-  hipStream_t s = nullptr;
-  hipStreamCreateWithFlags(&s, hipStreamNonBlocking);
+  hipStream_t own_stream = nullptr;
+  hipStreamCreateWithFlags(&own_stream, hipStreamNonBlocking);
   hipSetDevice(0);
+  hipStream_t s = own_stream;
+  if (!strcmp(what, "null stream")) s = nullptr;
+  if (!strcmp(what, "legacy stream")) s = hipStreamLegacy;
+  if (!strcmp(what, "per-thread stream")) s = hipStreamPerThread;
   hipMemPool_t def = nullptr, own = nullptr;
   hipDeviceGetDefaultMemPool(&def, dev);
   const hipMemPoolProps props{hipMemAllocationTypePinned, {hipMemLocationTypeDevice, dev}};
@@ -306,7 +310,7 @@ bool pool_case(const char *what)
   else ok = ok && emu_last_pool != def && emu_last_pool->threshold > 0;  // the library's
   hipDeviceSetMemPool(dev, def);
   hipMemPoolSetAttribute(def, hipMemPoolAttrReleaseThreshold, &none);
-  hipStreamDestroy(s);
+  hipStreamDestroy(own_stream);
   return ok;
 }
 
@@ -395,7 +399,8 @@ int main(int argc, char **argv)
   cases.push_back({"refused launch, deep spatial build", [] { return refused_spatial_build_case(110, 2, true); }});
   cases.push_back({"refused launch, sorted query", [] { return refused_sorted_query_case(); }});
   for (const char *what : {"nothing chosen", "stream of another device", "a current pool",
-                           "a default pool that keeps", "nothing chosen"})
+                           "a default pool that keeps", "null stream", "legacy stream",
+                           "per-thread stream", "nothing chosen"})
     cases.push_back({std::string("memory pool, ") + what, [=] { return pool_case(what); }});
   for (int nq : {1, 63, 64, 65})
     for (int flags : {CUKD_QUERY_SORT, CUKD_QUERY_AUTOTUNE, CUKD_QUERY_SORT | CUKD_QUERY_AUTOTUNE})

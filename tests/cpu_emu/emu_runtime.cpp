@@ -328,6 +328,7 @@ hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned)
   return hipSuccess;
 }
 hipError_t hipStreamDestroy(hipStream_t s) { delete s; return hipSuccess; }
+// like the runtime's, not for the handles hipStreamLegacy and hipStreamPerThread
 hipError_t hipStreamGetDevice(hipStream_t s, hipDevice_t *d)
 {
   *d = s ? s->device : emu_device;
@@ -355,8 +356,8 @@ hipError_t hipMallocFromPoolAsync(void **p, size_t n, hipMemPool_t pool, hipStre
 }
 hipError_t hipMallocAsync(void **p, size_t n, hipStream_t s)
 {
-  int d;
-  hipStreamGetDevice(s, &d);
+  int d = emu_device;
+  if (s != hipStreamLegacy && s != hipStreamPerThread) hipStreamGetDevice(s, &d);
   return hipMallocFromPoolAsync(p, n, emu_pools[d], s);
 }
 hipError_t hipDeviceGetAttribute(int *v, hipDeviceAttribute_t, int) { *v = 4; return hipSuccess; }

@@ -43,6 +43,8 @@ typedef struct {
   hipMemLocation location;
 } hipMemPoolProps;
 #define hipStreamNonBlocking 1
+#define hipStreamLegacy ((hipStream_t)1)
+#define hipStreamPerThread ((hipStream_t)2)
 #define hipEventDisableTiming 2
 #define hipHostMallocDefault 0
 

@@ -52,3 +52,17 @@ def test_default_pool_with_a_threshold_serves(hip):
     finally:
         attr(ATTR_RELEASE_THRESHOLD, 0)
     assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("stream", [0, 1, 2])  # null, hipStreamLegacy, hipStreamPerThread
+def test_stock_streams(stream):
+    lay = ck.float_points(3)
+    pts = torch.from_numpy(datagen.uniform(20_000, 3, 4)).cuda()
+    want = pts.clone()
+    ck.buildTree(want, lay)
+    torch.cuda.synchronize()
+    rc = ck.lib().cukd_build_tree(ctypes.c_void_p(pts.data_ptr()), len(pts), ctypes.byref(lay),
+                                  ck.BUILDER_DEFAULT, None, ctypes.c_void_p(stream), None)
+    assert rc == 0, ck.lib().cukd_last_error()
+    torch.cuda.synchronize()
+    assert torch.equal(pts, want)
