@@ -1095,7 +1095,7 @@ def main():
                      "algorithmic_bytes": "queries, results and the node visits of the "
                                           "reference's traversal, which is what achieved and "
                                           "frac are defined by; the kernel prunes by box and "
-                                          "moves fewer (traffic: what it moves)",
+                                          "makes fewer visits (traffic: the bytes it moves)",
                      "traffic_achieved": (None if traffic is None else
                                           round(traffic / (kernel_ms / 1e3) / 1e9, 2)),
                      "traffic_frac": (None if traffic is None else
